@@ -59,26 +59,56 @@ __device__ __forceinline__ float input_recip(const Cq4View& w, uint32_t k) {
     return 1.0f;
 }
 
-// Stores the code-basis value x of (row, k): as fp32 into out[row][k], or, when xs is set
-// (the MFMA path, K % 64 == 0), as its three exact bf16 limbs in the limb layout
-// [M][K/64][3][64] that cq4_gemm_mfma_kernel copies to LDS.
-__device__ __forceinline__ void store_code(float* out, uint16_t* xs, uint32_t K, size_t row, uint32_t k, float x) {
-    if (xs == nullptr) {
+// Limb layouts of the code-basis activations (each value as three exact bf16 limbs), chosen with
+// the GEMM that reads them. Values come in runs of eight consecutive k, 16 bytes per limb.
+//   kLimbsTile (cq4_gemm_pipe_kernel, cq4_gemm_mfma_kernel): [M][K/64][3][64], copied to LDS;
+//   v = 1, 2 or 4 (cq4_gemm_batch_kernel): [ceil(M/16)][K/32][3][64 lanes][8], the A operands of
+//     v_mfma_f32_16x16x32_bf16 as they are loaded, lane 16 q + row % 16. A step takes from lane
+//     quarter q the run t of the q-th v-run chunk of a 32 v-value unit (k = 32 v unit + 8 v q + 8 t),
+//     so that a lane's packed indices of a unit's v steps are 4 v contiguous bytes.
+// `panel` permutes a run into the order in which 4-row panels hold it: k % 8 = 0, 4, 1, 5, 2, 6, 3, 7.
+constexpr uint32_t kLimbsTile = 0;
+
+struct Cq4LimbOut {
+    uint16_t* xs;     // nullptr: fp32 rows are written instead
+    uint32_t layout;  // kLimbsTile or v
+    bool panel;
+};
+
+// Offset, in values, of limb 0 of the run holding (row, k); limb li is li * limb_stride further.
+__host__ __device__ __forceinline__ size_t limb_run(uint32_t layout, uint32_t K, size_t row, uint32_t k) {
+    if (layout == kLimbsTile) return (row * (K >> 6) + (k >> 6)) * (3 * 64) + (k & 56);
+    const uint32_t v = layout, vs = static_cast<uint32_t>(__builtin_ctz(v));
+    const uint32_t unit = k >> (5 + vs), run = (k >> 3) & (4 * v - 1);  // run of the unit
+    const size_t step = (row >> 4) * (K >> 5) + unit * v + (run & (v - 1));
+    return step * (3 * 512) + ((run >> vs) * 16 + (row & 15)) * 8;
+}
+__host__ __device__ __forceinline__ uint32_t limb_stride(uint32_t layout) { return layout == kLimbsTile ? 64 : 512; }
+// Position within its run of the value k.
+__host__ __device__ __forceinline__ uint32_t limb_slot(bool panel, uint32_t k) {
+    return panel ? 2 * (k & 3) + ((k >> 2) & 1) : (k & 7);
+}
+
+// Stores the code-basis value x of (row, k): as fp32 into out[row][k], or, when lo.xs is set, as its
+// three exact bf16 limbs in that layout.
+__device__ __forceinline__ void store_code(float* out, const Cq4LimbOut& lo, uint32_t K, size_t row, uint32_t k, float x) {
+    if (lo.xs == nullptr) {
         out[row * K + k] = x;
         return;
     }
     uint32_t b[3];
     split_bf16_limbs(x, b);
-    uint16_t* d = xs + (row * (K >> 6) + (k >> 6)) * (3 * 64) + (k & 63);
+    uint16_t* d = lo.xs + limb_run(lo.layout, K, row, k) + limb_slot(lo.panel, k);
+    const uint32_t stride = limb_stride(lo.layout);
     d[0] = static_cast<uint16_t>(b[0]);
-    d[64] = static_cast<uint16_t>(b[1]);
-    d[128] = static_cast<uint16_t>(b[2]);
+    d[stride] = static_cast<uint16_t>(b[1]);
+    d[2 * stride] = static_cast<uint16_t>(b[2]);
 }
 
 // Hadamard basis: grid (num_groups, M), group_size / 2 threads; thread t owns
 // elements t and t + gs/2 on load and store and butterfly t at every stage.
 __global__ __launch_bounds__(128) void cq4_transform_hadamard_kernel(Cq4View w, const uint16_t* __restrict__ a,
-                                                                     float* __restrict__ out, uint16_t* __restrict__ xs) {
+                                                                     float* __restrict__ out, Cq4LimbOut lo) {
     __shared__ float v[256];
     const uint32_t gs = w.group_size, half = gs >> 1;
     const uint32_t g = blockIdx.x, m = blockIdx.y, t = threadIdx.x;
@@ -104,7 +134,7 @@ __global__ __launch_bounds__(128) void cq4_transform_hadamard_kernel(Cq4View w, 
         // an out-of-range entry is masked into the group (the host entry point rejects it)
         const uint32_t src = w.permutation ? (w.permutation[j] & (gs - 1)) : j;
         const float sign = w.right_signs ? static_cast<float>(w.right_signs[src]) : 1.0f;
-        store_code(out, xs, w.K, m, g * gs + j, v[src] * inv * sign);
+        store_code(out, lo, w.K, m, g * gs + j, v[src] * inv * sign);
     }
 }
 
@@ -117,7 +147,7 @@ __global__ __launch_bounds__(128) void cq4_transform_hadamard_kernel(Cq4View w, 
 // above. Four wavefronts per workgroup cover four consecutive (row, group) pairs.
 template <int E>
 __global__ __launch_bounds__(256) void cq4_transform_hadamard_wave_kernel(Cq4View w, const uint16_t* __restrict__ a,
-                                                                          float* __restrict__ out, uint16_t* __restrict__ xs,
+                                                                          float* __restrict__ out, Cq4LimbOut lo,
                                                                           uint32_t pairs) {
     constexpr uint32_t gs = 64 * E;
     const uint32_t lane = threadIdx.x & 63;
@@ -190,7 +220,7 @@ __global__ __launch_bounds__(256) void cq4_transform_hadamard_wave_kernel(Cq4Vie
             }
         }
         const float sign = w.right_signs ? static_cast<float>(rs[i]) : 1.0f;
-        store_code(out, xs, w.K, pair / w.num_groups, g * gs + j, x * inv * sign);
+        store_code(out, lo, w.K, pair / w.num_groups, g * gs + j, x * inv * sign);
     }
 }
 
@@ -211,7 +241,7 @@ __device__ __forceinline__ float lane_xor(float v) {
     return __int_as_float(r);
 }
 
-// Hadamard basis written straight as bf16 limbs for the MFMA GEMM (group size GS = 64, 128 or 256;
+// Hadamard basis written straight as bf16 limbs for the MFMA GEMM (group size GS = 32 to 256;
 // activations and scales 16-byte aligned, signs 8-byte aligned): one wavefront per 512 consecutive
 // values of a row, lane l holding values 8 l .. 8 l + 7, so every load and limb store is 16 bytes
 // per lane. Butterflies of stride 1, 2 and 4 pair a lane's own values and strides 8 .. GS / 2 pair
@@ -224,10 +254,10 @@ __device__ __forceinline__ float lane_xor(float v) {
 // With xcd_rows set (the GEMM's row tiles a multiple of 8), workgroup b works on the rows of 64-row
 // tiles t with t % 8 == b % 8: workgroups run on XCD b % 8, and the GEMM reads row tile t on XCD
 // t % 8, so each row's limbs are written through the L2 that later serves them.
-template <int GS>
+template <int GS, bool TILE>
 __global__ __launch_bounds__(256) void cq4_transform_hadamard_limbs_kernel(Cq4View w, const uint16_t* __restrict__ a,
-                                                                           uint16_t* __restrict__ xs, uint32_t M,
-                                                                           uint32_t chunks, bool xcd_rows) {
+                                                                           Cq4LimbOut lo, uint32_t M, uint32_t chunks,
+                                                                           bool xcd_rows) {
     __shared__ float gather[4][512];
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     uint32_t row, chunk;
@@ -293,7 +323,7 @@ __global__ __launch_bounds__(256) void cq4_transform_hadamard_limbs_kernel(Cq4Vi
     };
     cross(std::integral_constant<int, 1>{});
     cross(std::integral_constant<int, 2>{});
-    cross(std::integral_constant<int, 4>{});
+    if constexpr (GS >= 64) cross(std::integral_constant<int, 4>{});
     if constexpr (GS >= 128) cross(std::integral_constant<int, 8>{});
     if constexpr (GS >= 256) cross(std::integral_constant<int, 16>{});
     const float inv = 1.0f / sqrtf(static_cast<float>(GS));
@@ -331,20 +361,22 @@ __global__ __launch_bounds__(256) void cq4_transform_hadamard_limbs_kernel(Cq4Vi
         for (int li = 0; li < 3; ++li) limb[li][e] = b[li];
     }
     if (live) {
-        uint16_t* d = xs + (static_cast<size_t>(row) * (K >> 6) + (k0 >> 6)) * (3 * 64) + (k0 & 63);
+        uint16_t* d = lo.xs + limb_run(TILE ? kLimbsTile : lo.layout, K, row, k0);
+        const uint32_t stride = limb_stride(TILE ? kLimbsTile : lo.layout);
 #pragma unroll
         for (int li = 0; li < 3; ++li) {
             u32x4 o;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = limb[li][2 * i] | (limb[li][2 * i + 1] << 16);
-            *reinterpret_cast<u32x4*>(d + 64 * li) = o;
+            for (int i = 0; i < 4; ++i)
+                o[i] = !TILE && lo.panel ? limb[li][i] | (limb[li][i + 4] << 16) : limb[li][2 * i] | (limb[li][2 * i + 1] << 16);
+            *reinterpret_cast<u32x4*>(d + stride * li) = o;
         }
     }
 }
 
 // Orthogonal basis: A_rot[m][i] = sum_k A[m][k] recip[k] R[k][i]; grid (ceil(K/256), M).
 __global__ __launch_bounds__(256) void cq4_transform_orthogonal_kernel(Cq4View w, const uint16_t* __restrict__ a,
-                                                                       float* __restrict__ out, uint16_t* __restrict__ xs) {
+                                                                       float* __restrict__ out, Cq4LimbOut lo) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, m = blockIdx.y;
     if (i >= w.K) return;
     const uint16_t* arow = a + static_cast<size_t>(m) * w.K;
@@ -352,7 +384,7 @@ __global__ __launch_bounds__(256) void cq4_transform_orthogonal_kernel(Cq4View w
     for (uint32_t k = 0; k < w.K; ++k)
         acc = fmaf(half_bits_to_float(arow[k]) * input_recip(w, k), half_bits_to_float(w.rotation[static_cast<size_t>(k) * w.K + i]),
                    acc);
-    store_code(out, xs, w.K, m, i, acc);
+    store_code(out, lo, w.K, m, i, acc);
 }
 
 // Index k of a row's LSB-first group (cactus_x86.cpp:24-43), any bits in 1..4.
@@ -1142,14 +1174,292 @@ __global__ __launch_bounds__(64 * kCq4PipeWaves) void cq4_gemm_pipe_kernel(Cq4Vi
     }
 }
 
+// Output (row, col) as IEEE arithmetic on the code-basis values and codebook themselves gives it:
+// fp32 sums over at most 32 values, folded with the norm in double, as cq4_gemm_kernel forms them.
+// The limb products cannot carry an infinity (it meets the zero limbs of its partner as NaN), so
+// the limb GEMMs take outputs that came out non-finite from here. Written for clarity: it runs only
+// for those.
+__device__ double cq4_ieee_output(const Cq4View& w, const Cq4LimbOut& lo, uint32_t row, uint32_t col, uint32_t gs,
+                                  uint32_t ng) {
+    const uint32_t stride = limb_stride(lo.layout);
+    double acc = 0.0;
+    for (uint32_t g = 0; g < ng; ++g) {
+        const size_t ni = lo.panel ? (static_cast<size_t>(col >> 2) * ng + g) * 4 + (col & 3)
+                                   : static_cast<size_t>(col) * ng + g;
+        const double norm = static_cast<double>(half_bits_to_float(w.norms[ni]));
+        for (uint32_t k0 = 0; k0 < gs; k0 += 32) {
+            float sum = 0.0f;
+            for (uint32_t e = 0; e < 32; ++e) {
+                const uint32_t k = g * gs + k0 + e;
+                const uint16_t* a = lo.xs + limb_run(lo.layout, w.K, row, k) + limb_slot(lo.panel, k);
+                const float x = (__uint_as_float(static_cast<uint32_t>(a[0]) << 16) +
+                                 __uint_as_float(static_cast<uint32_t>(a[stride]) << 16)) +
+                                __uint_as_float(static_cast<uint32_t>(a[2 * stride]) << 16);
+                uint32_t code;
+                if (lo.panel) {
+                    const uint8_t b = w.packed[static_cast<size_t>(col >> 2) * (2 * static_cast<size_t>(w.K)) +
+                                               static_cast<size_t>(k >> 3) * 16 + (col & 3) * 4 + (k & 3)];
+                    code = (k & 4) ? b >> 4 : b & 0xFu;
+                } else {
+                    const uint8_t b = w.packed[static_cast<size_t>(col) * (w.K >> 1) + (k >> 1)];
+                    code = (k & 1) ? b >> 4 : b & 0xFu;
+                }
+                sum = fmaf(x, half_bits_to_float(w.codebook[code & ((1u << w.bits) - 1u)]), sum);
+            }
+            acc = fma(norm, static_cast<double>(sum), acc);
+        }
+    }
+    return acc;
+}
+
+// Batches below the tiled kernel's 64-row tiles, panels and expanded indices of any row count:
+// group size a multiple of 32. At 8 x 4096 -> 4096 (8.4 MB of indices) the GEMM takes 8.3 us traced,
+// of which a SIMD issues for ~4 (1129 VALU instructions, 192 MFMAs of 16 cycles); the rest is the
+// latency of the first loads, so the work is cut for wavefronts in flight: a workgroup owns 16 columns
+// and 16 RB rows, its W wavefronts take four-step quads of K in turn (a step is 32 values: one
+// v_mfma_f32_16x16x32_bf16 per limb product), and their float64 sums are added through LDS in
+// wavefront order. Everything stays in registers:
+//   - lane (j = lane % 16, q = lane / 16) loads the packed indices of column j that its MFMA slots
+//     take. LSB-first packing: a unit of V steps is 32 V values of a column, of which lane quarter q
+//     takes the q-th 8 V in one 4 V-byte load (V = 4 for groups of 128 and more: a column's
+//     quarters read 64 contiguous bytes, where one word per step would take four passes over the
+//     same lines; V = 2 and 1 for groups of 64 and 32, since a step stays inside one group). Panels:
+//     step s reads words 4 s .. 4 s + 3 of a panel, 64 contiguous bytes for its four columns;
+//   - the transform wrote the activations in the order of the A operands (limb_run), so a step's
+//     limbs are three fully coalesced 1 KiB loads, from L2; rows past M read nothing (their lanes'
+//     offsets lie past the buffer) and are zero;
+//   - a step decodes its eight indices through a 256-entry table per codebook limb (two codes per
+//     byte, as in cq4_gemm_pipe_kernel; 16 copies of every word, which take the bank conflicts out,
+//     changed nothing), runs its six products smallest first into P from zero and
+//     folds acc += norm * P in float64: 32-value fp32 sums, as everywhere here;
+//   - the loads of quad i + 1 are issued during quad i (indices and norms before it, limbs as their
+//     registers are read).
+constexpr int kBufferWord3 = 0x00020000;      // buffer resource word 3: 32-bit data format
+constexpr uint32_t kCq4BatchMaxK = 1u << 23;  // a 16-row block's limbs end below the offsets that mean "past" (2^30)
+
+template <int V, bool INTER, int RB, int W>
+__global__ __launch_bounds__(64 * W) void cq4_gemm_batch_kernel(Cq4View w, Cq4LimbOut lo, uint16_t* __restrict__ c,
+                                                               uint32_t M, uint32_t gs, uint32_t ng,
+                                                               uint32_t group_shift) {
+    static_assert(!INTER || V == 1, "panels are read in K order");
+    constexpr int kRing = RB == 1 ? 4 : 2;  // steps of limbs in flight
+    __shared__ uint32_t lut[2][256];
+    __shared__ double red[W][RB * 4][64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, q = lane >> 4;
+    const int K = static_cast<int>(w.K), N = static_cast<int>(w.N);
+    const int S = K >> 5;          // steps
+    const int Q = (S + 3) >> 2;    // quads of steps
+    const int n0 = static_cast<int>(blockIdx.x) * 16;
+    const int m0 = static_cast<int>(blockIdx.y) * 16 * RB;
+
+    // The tile's columns and norms are contiguous in both layouts; columns past N lie past the range.
+    const int cols = min(16, N - n0);
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(w.packed) + static_cast<size_t>(n0) * (K >> 1), 0, cols * (K >> 1), kBufferWord3);
+    const __amdgpu_buffer_rsrc_t rn = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(w.norms) + static_cast<size_t>(n0) * ng, 0, cols * static_cast<int>(ng) * 2, kBufferWord3);
+    const uint32_t woff = INTER ? (j >> 2) * 2 * K + q * 16 + (j & 3) * 4 : j * (K >> 1) + q * 4 * V;
+    const uint32_t noff = INTER ? ((j >> 2) * ng * 4 + (j & 3)) * 2 : j * ng * 2;
+    __amdgpu_buffer_rsrc_t rx[RB];
+    uint32_t xoff[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+        const int r0 = m0 + 16 * rb;
+        const int live = static_cast<int>(M) - r0;  // rows of this block (may be <= 0)
+        rx[rb] = __builtin_amdgcn_make_buffer_rsrc(
+            lo.xs + static_cast<size_t>(live > 0 ? r0 >> 4 : 0) * S * (3 * 512), 0, S * 3072, kBufferWord3);
+        xoff[rb] = j < live ? static_cast<uint32_t>(lane) * 16u : 0x40000000u;
+    }
+
+    struct Quad {
+        uint32_t w[4];
+        uint16_t nb[4];
+    };
+    // A quad past the last reads nothing; a step past the last (only with V = 1 or 2) is not computed.
+    auto load_quad = [&](Quad& d, int qi) {
+        const uint32_t past = qi < Q ? 0u : 0x80000000u;
+        if constexpr (V == 4) {
+            const u32x4 t = __builtin_amdgcn_raw_buffer_load_b128(rw, woff + qi * 64 + past, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d.w[i] = t[i];
+            d.nb[0] = __builtin_amdgcn_raw_buffer_load_b16(rn, noff + ((qi * 128) >> group_shift) * 2 + past, 0, 0);
+        } else if constexpr (V == 2) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int u = 2 * qi + h;
+                const auto t = __builtin_amdgcn_raw_buffer_load_b64(rw, woff + u * 32 + past, 0, 0);
+                d.w[2 * h] = t[0];
+                d.w[2 * h + 1] = t[1];
+                d.nb[2 * h] = __builtin_amdgcn_raw_buffer_load_b16(rn, noff + ((u * 64) >> group_shift) * 2 + past, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int st = 4 * qi + t;
+                const uint32_t g = static_cast<uint32_t>(st * 32) >> group_shift;
+                d.w[t] = __builtin_amdgcn_raw_buffer_load_b32(rw, woff + st * (INTER ? 64 : 16) + past, 0, 0);
+                d.nb[t] = __builtin_amdgcn_raw_buffer_load_b16(rn, noff + g * (INTER ? 8 : 2) + past, 0, 0);
+            }
+        }
+    };
+    auto norm_of = [](const Quad& d, int t) { return d.nb[V == 4 ? 0 : (V == 2 ? t & 2 : t)]; };
+    struct Limbs {
+        u32x4 a[RB][3];
+    };
+    auto load_limbs = [&](Limbs& d, int qi, int t) {
+        const uint32_t so = qi < Q ? static_cast<uint32_t>(4 * qi + t) * 3072u : 0x80000000u;  // past: reads nothing
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int li = 0; li < 3; ++li)
+                d.a[rb][li] = __builtin_amdgcn_raw_buffer_load_b128(rx[rb], xoff[rb] + so + li * 1024, 0, 0);
+    };
+
+    Quad quad[2];
+    Limbs ring[kRing];
+    load_quad(quad[0], wv);
+#pragma unroll
+    for (int t = 0; t < kRing; ++t) load_limbs(ring[t], wv, t);
+    for (int e = tid; e < 512; e += 64 * W) {  // the byte tables: limb e / 256, byte e % 256
+        auto limb = [&](uint32_t code) {
+            const float v = half_bits_to_float(w.codebook[code & ((1u << w.bits) - 1u)]);
+            const uint32_t hi = __float_as_uint(v) & 0xFFFF0000u;
+            return e < 256 ? hi >> 16 : __float_as_uint(v - __uint_as_float(hi)) >> 16;
+        };
+        lut[e >> 8][e & 255] = limb(e & 15) | (limb((e >> 4) & 15) << 16);
+    }
+    __syncthreads();
+
+    double acc[RB][4];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[rb][i] = 0.0;
+    const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    typedef __attribute__((address_space(3))) const volatile uint32_t lds_word;
+    lds_word* lutw = (lds_word*)(&lut[0][0]);
+    auto run_quad = [&](const Quad& cur, Quad& nxt, int qi) {
+        load_quad(nxt, qi + W);
+        static_for<4>([&](auto tc) {
+            constexpr int t = decltype(tc)::value;
+            Limbs& x = ring[t % kRing];
+            if (V == 4 || 4 * qi + t < S) {  // uniform
+                u32x4 hi, lw;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t b = (cur.w[t] >> (8 * i)) & 0xFFu;
+                    hi[i] = lutw[b];
+                    lw[i] = lutw[256 + b];
+                }
+                const bf16x8 bh = __builtin_bit_cast(bf16x8, hi), bl = __builtin_bit_cast(bf16x8, lw);
+                const double nv = static_cast<double>(half_bits_to_float(norm_of(cur, t)));
+                f32x4_t P[RB];
+                auto product = [&](int li, const bf16x8& b, bool first) {
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+                        P[rb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x.a[rb][li]), b,
+                                                                        first ? zero : P[rb], 0, 0, 0);
+                };
+                product(2, bl, true);
+                product(1, bl, false);
+                product(2, bh, false);
+                product(0, bl, false);
+                product(1, bh, false);
+                product(0, bh, false);
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[rb][i] = fma(nv, static_cast<double>(P[rb][i]), acc[rb][i]);
+            }
+            // this slot's next step, kRing further on
+            if constexpr (t + kRing < 4)
+                load_limbs(x, qi, t + kRing);
+            else
+                load_limbs(x, qi + W, t + kRing - 4);
+        });
+    };
+    for (int qi = wv; qi < Q; qi += 2 * W) {
+        run_quad(quad[0], quad[1], qi);
+        if (qi + W < Q) run_quad(quad[1], quad[0], qi + W);  // uniform
+    }
+
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[wv][rb * 4 + i][lane] = acc[rb][i];
+    __syncthreads();
+    for (int e = tid; e < RB * 256; e += 64 * W) {
+        const int slot = e >> 6, l = e & 63;
+        const int row = m0 + 16 * (slot >> 2) + 4 * (l >> 4) + (slot & 3), col = n0 + (l & 15);
+        if (row >= static_cast<int>(M) || col >= N) continue;
+        double s = red[0][slot][l];
+#pragma unroll
+        for (int v = 1; v < W; ++v) s += red[v][slot][l];
+        if (!__builtin_isfinite(s)) s = cq4_ieee_output(w, lo, row, col, gs, ng);  // rare
+        c[static_cast<size_t>(row) * N + col] = double_to_half_bits(s);
+    }
+}
+
+// 1- to 3-bit LSB-packed indices (group size a multiple of 32, so the whole matrix is one bit
+// string) rewritten as 4-bit ones for the limb GEMMs: a thread expands 32 indices, BITS words into
+// four. (Decoding other widths in the GEMMs would put their bit extraction into every row tile.)
+template <int BITS>
+__global__ __launch_bounds__(256) void cq4_expand_kernel(const uint32_t* __restrict__ packed, u32x4* __restrict__ out,
+                                                         size_t runs) {
+    const size_t e = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;  // 32-index run
+    if (e >= runs) return;
+    uint32_t in[BITS + 1];
+#pragma unroll
+    for (int i = 0; i < BITS; ++i) in[i] = packed[e * BITS + i];
+    in[BITS] = 0u;  // read only past the last bit
+    u32x4 o;
+#pragma unroll
+    for (int wd = 0; wd < 4; ++wd) {
+        uint32_t r = 0u;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const int bit = (8 * wd + t) * BITS;
+            const uint64_t two = (static_cast<uint64_t>(in[bit / 32 + 1]) << 32) | in[bit / 32];
+            r |= (static_cast<uint32_t>(two >> (bit % 32)) & ((1u << BITS) - 1u)) << (4 * t);
+        }
+        o[wd] = r;
+    }
+    out[e] = o;
+}
+
 // A null pointer counts as aligned (the array is absent).
 bool aligned(const void* p, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(p) & (bytes - 1)) == 0; }
 
-bool cq4_uses_mfma(const Cq4View& w, uint32_t m) {
+// How a call that the fused GEMV does not take runs.
+struct Cq4Plan {
+    enum Kind { kVector, kTile, kBatch } kind;  // fp32 activations on the VALU GEMMs, or a limb GEMM
+    uint32_t layout;                            // limb layout (kTile, kBatch)
+    size_t limb_bytes;                          // activations in the workspace
+    size_t code_bytes;                          // indices expanded to 4 bits behind them, or 0
+};
+
+// The limb GEMMs need steps of 32 values that stay inside one norm group. From 32 rows on the tiled
+// kernels take the reference benchmark's format (4-bit LSB-first, K % 64 == 0). cq4_gemv_kernel keeps
+// one row, and two or three of fewer than 2048 columns, where its four columns per workgroup spread
+// over more CUs than the batch kernel's sixteen (us per call at K = 8192: 1 x 512 14.1 against 17.9,
+// 2 x 1024 16.2 against 17.9, 3 x 2048 19.2 against 18.3, 2 x 8192 47 against 30). Everything else goes to
+// the batch kernel (8 x 4096 -> 4096 in panels: 13.5 us against 171 on the VALU GEMM, whose 32
+// workgroups run one thread per column and 4 rows; 3-bit indices at 5 x 2048 -> 2048 13.8 against 497).
+Cq4Plan cq4_plan(const Cq4View& w, uint32_t m) {
     const bool orth = (w.flags & kCq4FlagOrthogonal) != 0;
     const uint32_t gs = orth ? w.K : w.group_size;
     const bool inter = (w.flags & kCq4FlagInterleaved4Row) != 0;
-    return m >= kCq4MfmaMinRows && w.bits == 4 && !inter && gs % 32 == 0 && w.K % 64 == 0;
+    const size_t values = static_cast<size_t>(m) * w.K;
+    if (m >= kCq4MfmaMinRows && w.bits == 4 && !inter && gs % 32 == 0 && w.K % 64 == 0)
+        return {Cq4Plan::kTile, kLimbsTile, values * 3 * sizeof(uint16_t), 0};
+    const bool gemv = w.bits == 4 && (m == 1 || (m <= 3 && w.N < 2048));
+    if (gs % 32 != 0 || w.K > kCq4BatchMaxK || gemv) return {Cq4Plan::kVector, 0, values * sizeof(float), 0};
+    Cq4Plan p{Cq4Plan::kBatch, inter || gs % 64 != 0 ? 1u : gs % 128 != 0 ? 2u : 4u, 0, 0};
+    p.limb_bytes = static_cast<size_t>((m + 15) / 16) * 16 * w.K * 3 * sizeof(uint16_t);  // a multiple of 256
+    if (w.bits < 4) p.code_bytes = static_cast<size_t>(w.N) * (w.K / 2);
+    return p;
 }
 
 // Decode-sized Hadamard calls: transform and GEMV in one launch (cq4_gemv_fused_kernel).
@@ -1174,22 +1484,42 @@ hipError_t launch_gemm(const Cq4View& w, const float* ap, uint16_t* c, uint32_t 
     return hipGetLastError();
 }
 
+template <int V, bool INTER>
+hipError_t launch_batch(const Cq4View& w, const Cq4LimbOut& lo, uint16_t* c, uint32_t m, uint32_t gs, uint32_t ng,
+                        hipStream_t stream) {
+    const uint32_t group_shift = ng == 1 ? 31 : static_cast<uint32_t>(__builtin_ctz(gs));  // gs is a power of two then
+    const uint32_t tiles_n = (w.N + 15) / 16, quads = (w.K / 32 + 3) / 4;
+    auto go = [&](auto rb, auto wv) {
+        constexpr int RB = decltype(rb)::value, W = decltype(wv)::value;
+        hipLaunchKernelGGL((cq4_gemm_batch_kernel<V, INTER, RB, W>), dim3(tiles_n, (m + 16 * RB - 1) / (16 * RB)),
+                           dim3(64 * W), 0, stream, w, lo, c, m, gs, ng, group_shift);
+        return hipGetLastError();
+    };
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    using I4 = std::integral_constant<int, 4>;
+    using I8 = std::integral_constant<int, 8>;
+    using I16 = std::integral_constant<int, 16>;
+    if (m <= 16) return tiles_n <= 512 && quads > 8 ? go(I1{}, I16{}) : quads > 4 ? go(I1{}, I8{}) : go(I1{}, I4{});
+    if (m <= 32) return quads > 4 ? go(I2{}, I8{}) : go(I2{}, I4{});
+    return quads > 4 ? go(I4{}, I8{}) : go(I4{}, I4{});
+}
+
 }  // namespace
 
 size_t cq4_workspace_bytes(const Cq4View& w, uint32_t m) {
     if (cq4_gemv_fused(w, m)) return 0;
-    const size_t values = static_cast<size_t>(m) * w.K;  // K % 64 == 0 on the MFMA path: no padding
-    return cq4_uses_mfma(w, m) ? values * 3 * sizeof(uint16_t) : values * sizeof(float);
+    const Cq4Plan p = cq4_plan(w, m);
+    return p.limb_bytes + p.code_bytes;
 }
 
 hipError_t launch_cq4_matmul(const Cq4View& w, const uint16_t* a, uint32_t m, uint16_t* c, void* workspace,
                              hipStream_t stream) {
-    // The transform writes the code-basis activations as fp32 rows, or, for the MFMA GEMM, directly as
-    // their bf16 limbs.
+    const bool orth = (w.flags & kCq4FlagOrthogonal) != 0;
+    const bool inter = (w.flags & kCq4FlagInterleaved4Row) != 0;
     if (cq4_gemv_fused(w, m)) {
         const dim3 grid((w.N + 3) / 4);
         const size_t lds = 2 * sizeof(float) * m * w.K;
-        const bool inter = (w.flags & kCq4FlagInterleaved4Row) != 0;
         const uint32_t gs = w.group_size, ng = w.num_groups;
         if (m == 1) {
             if (inter) hipLaunchKernelGGL((cq4_gemv_fused_kernel<1, true>), grid, dim3(256), lds, stream, w, a, c, m, gs, ng);
@@ -1200,58 +1530,80 @@ hipError_t launch_cq4_matmul(const Cq4View& w, const uint16_t* a, uint32_t m, ui
         }
         return hipGetLastError();
     }
-    const bool mfma = cq4_uses_mfma(w, m);
-    float* ap = mfma ? nullptr : static_cast<float*>(workspace);
-    uint16_t* xs = mfma ? static_cast<uint16_t*>(workspace) : nullptr;
-    const bool orth = (w.flags & kCq4FlagOrthogonal) != 0;
+    // The transform writes the code-basis activations as fp32 rows, or, for the limb GEMMs, directly as
+    // their bf16 limbs.
+    const Cq4Plan plan = cq4_plan(w, m);
+    const bool limbs = plan.kind != Cq4Plan::kVector;
+    float* ap = limbs ? nullptr : static_cast<float*>(workspace);
+    const Cq4LimbOut lo{limbs ? static_cast<uint16_t*>(workspace) : nullptr, plan.layout, inter};
     const uint32_t gs = orth ? w.K : w.group_size, ng = orth ? 1 : w.num_groups;
     if (orth) {
         hipLaunchKernelGGL(cq4_transform_orthogonal_kernel, dim3((w.K + 255) / 256, m), dim3(256), 0, stream, w, a,
-                           ap, xs);
-    } else if (mfma && (w.group_size == 64 || w.group_size == 128 || w.group_size == 256) && aligned(a, 16) &&
-               aligned(w.input_scale_recip, 16) && aligned(w.input_scale, 16) && aligned(w.left_signs, 8) &&
-               aligned(w.right_signs, 8) && aligned(w.permutation, 16)) {
+                           ap, lo);
+    } else if (limbs && aligned(a, 16) && aligned(w.input_scale_recip, 16) && aligned(w.input_scale, 16) &&
+               aligned(w.left_signs, 8) && aligned(w.right_signs, 8) && aligned(w.permutation, 16)) {
         const uint32_t chunks = (w.K + 511) / 512;
         const uint32_t tiles_m = (m + kCq4Tile - 1) / kCq4Tile;
-        const bool xcd_rows = tiles_m % 8 == 0;  // the GEMM then reads row tile t on XCD t % 8
+        // the tiled GEMM then reads row tile t on XCD t % 8
+        const bool xcd_rows = plan.kind == Cq4Plan::kTile && tiles_m % 8 == 0;
         // XCD lane x holds tiles_m / 8 row tiles of 64 rows (the last may be partial)
         const dim3 grid(xcd_rows ? 8 * ((tiles_m / 8 * kCq4Tile * chunks + 3) / 4) : (m * chunks + 3) / 4);
-        if (w.group_size == 64)
-            hipLaunchKernelGGL(cq4_transform_hadamard_limbs_kernel<64>, grid, dim3(256), 0, stream, w, a, xs, m, chunks,
-                               xcd_rows);
-        else if (w.group_size == 128)
-            hipLaunchKernelGGL(cq4_transform_hadamard_limbs_kernel<128>, grid, dim3(256), 0, stream, w, a, xs, m, chunks,
-                               xcd_rows);
-        else
-            hipLaunchKernelGGL(cq4_transform_hadamard_limbs_kernel<256>, grid, dim3(256), 0, stream, w, a, xs, m, chunks,
-                               xcd_rows);
+        auto go = [&](auto group, auto tile) {
+            hipLaunchKernelGGL((cq4_transform_hadamard_limbs_kernel<decltype(group)::value, decltype(tile)::value>), grid,
+                               dim3(256), 0, stream, w, a, lo, m, chunks, xcd_rows);
+        };
+        auto by_group = [&](auto tile) {
+            if (w.group_size == 32) go(std::integral_constant<int, 32>{}, tile);
+            else if (w.group_size == 64) go(std::integral_constant<int, 64>{}, tile);
+            else if (w.group_size == 128) go(std::integral_constant<int, 128>{}, tile);
+            else go(std::integral_constant<int, 256>{}, tile);
+        };
+        if (plan.kind == Cq4Plan::kTile) by_group(std::true_type{});
+        else by_group(std::false_type{});
     } else if (w.group_size == 64 || w.group_size == 128 || w.group_size == 256) {
         const uint32_t pairs = m * w.num_groups;
         const dim3 grid((pairs + 3) / 4);
         if (w.group_size == 64)
-            hipLaunchKernelGGL(cq4_transform_hadamard_wave_kernel<1>, grid, dim3(256), 0, stream, w, a, ap, xs, pairs);
+            hipLaunchKernelGGL(cq4_transform_hadamard_wave_kernel<1>, grid, dim3(256), 0, stream, w, a, ap, lo, pairs);
         else if (w.group_size == 128)
-            hipLaunchKernelGGL(cq4_transform_hadamard_wave_kernel<2>, grid, dim3(256), 0, stream, w, a, ap, xs, pairs);
+            hipLaunchKernelGGL(cq4_transform_hadamard_wave_kernel<2>, grid, dim3(256), 0, stream, w, a, ap, lo, pairs);
         else
-            hipLaunchKernelGGL(cq4_transform_hadamard_wave_kernel<4>, grid, dim3(256), 0, stream, w, a, ap, xs, pairs);
+            hipLaunchKernelGGL(cq4_transform_hadamard_wave_kernel<4>, grid, dim3(256), 0, stream, w, a, ap, lo, pairs);
     } else {
         // group_size / 2 threads (one for a group of 1, whose transform is the identity)
         hipLaunchKernelGGL(cq4_transform_hadamard_kernel, dim3(w.num_groups, m), dim3(w.group_size > 1 ? w.group_size / 2 : 1),
-                           0, stream, w, a, ap, xs);
+                           0, stream, w, a, ap, lo);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const bool inter = (w.flags & kCq4FlagInterleaved4Row) != 0;
-    if (mfma) {
+    if (plan.kind == Cq4Plan::kTile) {
         const uint32_t tiles_m = (m + kCq4Tile - 1) / kCq4Tile, tiles_n = (w.N + kCq4Tile - 1) / kCq4Tile;
         // the pipelined kernel copies the tile's norms in 4-byte units
         if (ng <= kCq4NormsMax && (static_cast<size_t>(w.N) * ng) % 2 == 0 && aligned(w.norms, 4))
             hipLaunchKernelGGL(cq4_gemm_pipe_kernel, dim3(tiles_m * tiles_n), dim3(64 * kCq4PipeWaves), 0, stream, w,
-                               xs, c, m, gs, ng, tiles_m);
+                               lo.xs, c, m, gs, ng, tiles_m);
         else
-            hipLaunchKernelGGL(cq4_gemm_mfma_kernel, dim3(tiles_m * tiles_n), dim3(256), 0, stream, w, xs, c, m, gs,
+            hipLaunchKernelGGL(cq4_gemm_mfma_kernel, dim3(tiles_m * tiles_n), dim3(256), 0, stream, w, lo.xs, c, m, gs,
                                ng, tiles_m);
         return hipGetLastError();
+    }
+    if (plan.kind == Cq4Plan::kBatch) {
+        Cq4View v = w;
+        if (plan.code_bytes) {
+            u32x4* codes = reinterpret_cast<u32x4*>(static_cast<char*>(workspace) + plan.limb_bytes);
+            const size_t runs = plan.code_bytes / 16;
+            const dim3 grid(static_cast<unsigned>((runs + 255) / 256));
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(w.packed);
+            if (w.bits == 1) hipLaunchKernelGGL(cq4_expand_kernel<1>, grid, dim3(256), 0, stream, src, codes, runs);
+            else if (w.bits == 2) hipLaunchKernelGGL(cq4_expand_kernel<2>, grid, dim3(256), 0, stream, src, codes, runs);
+            else hipLaunchKernelGGL(cq4_expand_kernel<3>, grid, dim3(256), 0, stream, src, codes, runs);
+            if ((e = hipGetLastError()) != hipSuccess) return e;
+            v.packed = reinterpret_cast<const uint8_t*>(codes);
+        }
+        if (inter) return launch_batch<1, true>(v, lo, c, m, gs, ng, stream);
+        if (plan.layout == 4) return launch_batch<4, false>(v, lo, c, m, gs, ng, stream);
+        if (plan.layout == 2) return launch_batch<2, false>(v, lo, c, m, gs, ng, stream);
+        return launch_batch<1, false>(v, lo, c, m, gs, ng, stream);
     }
     if (m <= 4 && w.bits == 4 && gs % 8 == 0) {
         const dim3 grid((w.N + 3) / 4);

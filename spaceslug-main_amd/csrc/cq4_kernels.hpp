@@ -26,8 +26,9 @@ struct Cq4View {
     const uint16_t* rotation;
 };
 
-// Device bytes launch_cq4_matmul needs for m rows: the code-basis activations, as m * K floats,
-// or on the MFMA path as their bf16 limbs (6 * m * K bytes).
+// Device bytes launch_cq4_matmul needs for m rows: the code-basis activations, as m * K floats or,
+// for the MFMA GEMMs, as their bf16 limbs (6 bytes a value; whole 16-row blocks for the batch
+// kernel), and behind them 1- to 3-bit indices expanded to 4 bits (N * K / 2 bytes).
 size_t cq4_workspace_bytes(const Cq4View& w, uint32_t m);
 
 // C[m][N] (fp16) = transform(A[m][K] fp16) x decode(W). `workspace` holds

@@ -264,3 +264,59 @@ def test_decode_call_in_a_hip_graph(session, gpu):
     g2.replay()
     torch.cuda.synchronize()
     assert torch.all(c64 == 1)
+
+
+# The batch kernel: steps of 32 values dealt in quads to 4, 8 or 16 wavefronts (odd quad counts, a
+# last quad of one to three steps with groups of 32 and 64), one, two and four 16-row blocks with
+# ragged rows, ragged 16-column tiles, panels, K % 64 != 0, and 1- to 3-bit indices expanded first.
+BATCH_CASES = [dict(bits=4, K=8192, N=20, group_size=128, m=1),
+               dict(bits=4, K=2176, N=33, group_size=128, signs=True, perm=True, scale="scale", m=16),
+               dict(bits=4, K=320, N=17, group_size=64, perm=True, m=5),
+               dict(bits=4, K=32, N=1, group_size=32, signs=True, m=6),
+               dict(bits=4, K=1248, N=50, group_size=32, signs=True, scale="scale", m=17),
+               dict(bits=4, K=96, N=40, group_size=32, m=70),
+               dict(bits=4, K=2048, N=36, group_size=256, interleaved=True, signs=True, perm=True, m=31),
+               dict(bits=4, K=1120, N=20, group_size=32, interleaved=True, m=8),
+               dict(bits=4, K=384, N=68, group_size=128, interleaved=True, scale="none", m=129),
+               dict(bits=4, K=160, N=24, group_size=160, interleaved=True, orthogonal=True, m=9),
+               dict(bits=4, K=192, N=24, group_size=192, orthogonal=True, m=3),
+               dict(bits=3, K=768, N=37, group_size=128, signs=True, m=40),
+               dict(bits=2, K=512, N=18, group_size=64, m=4),
+               dict(bits=1, K=96, N=21, group_size=32, m=33)]
+
+
+@pytest.mark.parametrize("case", range(len(BATCH_CASES)))
+def test_random_matrices_batch(session, gpu, case):
+    kw = dict(BATCH_CASES[case])
+    m = kw.pop("m")
+    rng = np.random.default_rng(1300 + case)
+    W = cq4.random_matrix(rng, **kw)
+    A = cq4.f16(rng.uniform(-1, 1, (m, W.K)))
+    check(session, W, A, m, f"batch {BATCH_CASES[case]} m={m}")
+
+
+@pytest.mark.parametrize("interleaved,K,gs,m", [(False, 256, 64, 6), (True, 256, 128, 6), (False, 128, 128, 20)])
+def test_batch_nonfinite_follows_ieee(session, gpu, interleaved, K, gs, m):
+    """Infinities and NaNs in the activations, a norm or the codebook: the batch kernel's limb products
+    cannot carry them, so every output's class (finite, +inf, -inf, NaN) is compared with double
+    arithmetic on the code-basis activations, which the Hadamard transform spreads over a group."""
+    rng = np.random.default_rng(41)
+    W = cq4.random_matrix(rng, bits=4, K=K, N=20, group_size=gs, interleaved=interleaved, signs=True)
+    W.codebook[3], W.codebook[9] = cq4.f16(np.array([0.0, -0.5]))  # a zero entry: inf * 0 is NaN
+    A = cq4.f16(rng.uniform(-1, 1, (m, K)))
+    A[1, 5] = 0x7C00            # +inf
+    A[2, 70 % K] = 0xFC00       # -inf
+    A[3, 1] = 0x7E00            # NaN
+    A[4, 2], A[4, 3] = 0x7C00, 0xFC00
+    for code in (None, 7):      # then also an infinite codebook entry
+        if code is not None:
+            W.codebook[code] = 0x7C00
+        got = run(session, W, A, m).view(np.float16).astype(np.float64)
+        with np.errstate(invalid="ignore"):
+            ref = cq4.matmul(W, A, m)
+        assert np.array_equal(np.isnan(got), np.isnan(ref)), code
+        assert np.array_equal(np.isposinf(got), np.isposinf(ref)), code
+        assert np.array_equal(np.isneginf(got), np.isneginf(ref)), code
+        ok = np.isfinite(ref)
+        assert ok.any() == (code is None)
+        assert np.all(np.abs(got[ok] - ref[ok]) <= 2.0 ** -11 * np.abs(ref[ok]) + 1e-5 * np.maximum(1, np.abs(ref[ok])))
