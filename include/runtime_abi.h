@@ -45,7 +45,8 @@
  *     (x in [-1, 1), scales in [0.5, 1.5); test_q4gemm.cpp:168-176), asserted for
  *     m = 1..32 at K up to 8192 (the decode GEMV up to K = 32768), and on x
  *     whose groups span 1e-30..1e30.
- *   - m > 32 (bf16 MFMA on x split exactly into three bf16 limbs; every product
+ *   - m > 32: shapes too small to fill the device's tile grids run as above; the
+ *     others (bf16 MFMA on x split exactly into three bf16 limbs; every product
  *     exact, one fp32 rounding per MFMA of each 32-value group sum, groups summed
  *     in double): the error grows like sqrt(K / 32). Stated tolerance
  *     6e-6 * sqrt(K / 32) on unit-range inputs (the KAT's ranges; asserted at
@@ -118,16 +119,16 @@ int spaceslug_q4gemm_lora(const float* x, const uint8_t* w_packed, const float* 
  * Enqueues only. Without LoRA, calls of up to 32 rows use no device memory
  * beyond their arguments; above 32 rows the three bf16 limbs of x (6 * m * k
  * bytes, m rounded up to a multiple of 16 on the 128 x 128 tiles) and any
- * K-split partial sums, and in LoRA calls the T = x * lora_a partials, live
- * in a library-owned device workspace that is allocated on first use and
+ * K-split partial sums, where the shape's kernel has them, and in LoRA calls
+ * the T = x * lora_a partials, live in a library-owned device workspace that is allocated on first use and
  * grown on demand (growth synchronises the device, steady state does not
  * allocate). Calls that share a device share that workspace; the library
  * orders them: a call on a stream other than the previous user's makes its
  * stream wait (on the GPU, hipStreamWaitEvent) for that user's kernels, and
- * host threads are serialised while enqueueing. A call that needs that
- * workspace returns SPACESLUG_ERR_UNSUPPORTED, enqueueing nothing, while
+ * host threads are serialised while enqueueing. A call above 32 rows or with
+ * LoRA returns SPACESLUG_ERR_UNSUPPORTED, enqueueing nothing, while
  * `stream` is being captured into a graph (the graph would keep an address a
- * later, larger call frees): capture a spaceslug_q4_chain or use
+ * later, larger call frees), whichever kernel it would run: capture a spaceslug_q4_chain or use
  * spaceslug_q4gemm_device_noalloc. */
 int spaceslug_q4gemm_device(const float* d_x, const uint8_t* d_w_packed, const float* d_w_scales,
                             float* d_y, uint32_t m, uint32_t n, uint32_t k, void* stream);
@@ -140,8 +141,8 @@ int spaceslug_q4gemm_device(const float* d_x, const uint8_t* d_w_packed, const f
  * arguments, contract and results as spaceslug_q4gemm_device, but the call allocates and
  * frees nothing: the scratch its kernels need (the bf16 limbs of x above 32 rows, K-split
  * partial sums) lives in one fixed array of SPACESLUG_Q4_NOALLOC_SCRATCH_BYTES per device,
- * held from module load until the process ends. A shape whose scratch would exceed it
- * returns 1 without enqueueing anything (the five workload shapes fit: 2048 x 4096 x 14336
+ * held from module load until the process ends. A shape whose limbs and partial sums would
+ * exceed it returns 1 without enqueueing anything, also where its kernel needs none (the five workload shapes fit: 2048 x 4096 x 14336
  * needs 48 MiB). Every call on a device shares that device's array and nothing in it needs
  * to start at zero; calls that overlap on one device (other streams, or threads) race on it,
  * so callers order them, e.g. on one stream. */

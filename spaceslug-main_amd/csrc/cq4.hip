@@ -17,24 +17,12 @@
 
 #include <cstdint>
 #include <type_traits>
-#include <utility>
 
 #include "cq4_kernels.hpp"
 #include "q4_device.hpp"
 
 namespace spaceslug {
 namespace {
-
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-
-// f(integral_constant<int, i>) for i = 0 .. N-1, unrolled at compile time.
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
 
 __device__ __forceinline__ float half_bits_to_float(uint16_t h) { return static_cast<float>(__builtin_bit_cast(_Float16, h)); }
 

@@ -1,7 +1,7 @@
 // MFMA int4 GEMM for more than 32 rows (prefill, LoRA projections, the reference's
 // 1024^3 bench shape). Two kernels: q4_gemm_wide_kernel, and q4_gemm_mid_kernel for
 // the shapes whose wide grid would need a K-split, each described at its definition.
-// (Up to 32 rows the exact small-batch GEMM of q4_small.hip runs instead.)
+// (Up to 32 rows, and for small grids above, the exact digit GEMMs of q4_small.hip run instead.)
 //
 // Replaces q4gemm.comp:61-175 (64x64 tile, LDS-staged dequantised B, 4x4 FMA
 // micro-tile per thread) with a CDNA4 design on the matrix cores:
@@ -27,7 +27,6 @@
 // epilogue sums them (lora_t_values) and adds scale * T[rows] * lb[:, cols] with the
 // same MFMA tile layout (r in the K slot) before the single store of y.
 #include <algorithm>
-#include <utility>
 
 #include "q4_device.hpp"
 #include "q4_kernels.hpp"
@@ -35,17 +34,6 @@
 
 namespace spaceslug {
 namespace {
-
-// Calls f(std::integral_constant<int, I>{}) for I = 0 .. N-1 in order (compile-time indices, so
-// register arrays indexed by I stay in registers).
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
 
 // Limbs per x value on the bf16 MFMA path.
 constexpr int kLimbs = 3;
@@ -913,7 +901,7 @@ size_t split_x_bf16_bytes(uint32_t m, uint32_t k) {
 }
 
 Q4Plan plan_q4gemm(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, uint32_t rank) {
-    Q4Plan plan{Q4Plan::kGemv, 1, 0, 0};
+    Q4Plan plan{Q4Plan::kGemv, 1, 0, 0, 0, 0};
     if (rank == 0 && gemv_takes(m, k)) return plan;
     const int groups = static_cast<int>(k / kGroup);
     size_t lora_bytes = 0;
@@ -921,9 +909,11 @@ Q4Plan plan_q4gemm(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, ui
         plan.t_splits = (groups + kLoraGroupsPerBlock - 1) / kLoraGroupsPerBlock;
         lora_bytes += align_up(static_cast<size_t>(plan.t_splits) * m * rank * sizeof(float));  // T partials
     }
+    const DigitTiles digits = plan_digit_tiles(dev, m, n, k);
     if (m <= 32) {
         plan.kind = Q4Plan::kDigits;
-        plan.workspace_bytes = lora_bytes;  // the T partials of a LoRA call; none otherwise
+        plan.tiles = digits.tiles;
+        plan.workspace_bytes = plan.contract_bytes = lora_bytes;  // the T partials of a LoRA call; none otherwise
         return plan;
     }
     plan.kind = Q4Plan::kWide;
@@ -940,16 +930,38 @@ Q4Plan plan_q4gemm(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, ui
     splits = (groups + per_split - 1) / per_split;
     plan.splits = splits;
     const size_t mid_tiles = static_cast<size_t>((m + kMidTile - 1) / kMidTile) * ((n + kMidTile - 1) / kMidTile);
+    // Time estimates in microseconds, fitted to 120 shapes (33 to 512 rows, 320 to 14336 columns, K = 64 to
+    // 14336; mid-size within 10%, wide within 15%): the launches and the pipeline's fill, then per 64
+    // values of K (mid-size), per group and round of workgroups (wide), and for a K-split the
+    // reduction's rounds of loads and the partial planes written and read.
+    float us;
     if (splits > 1 && rank == 0 && k % 64 == 0 && groups <= kMidGroupsMax &&
         mid_tiles <= static_cast<size_t>(dev.cu_count)) {
         plan.kind = Q4Plan::kMid;  // whole K per 64 x 64 tile: no partials, no reduction launch
         plan.splits = 1;
         plan.workspace_bytes = align_up(static_cast<size_t>(m) * k * kLimbs * sizeof(uint16_t));  // x limbs
-        return plan;
+        us = 10.0f + 0.6f * static_cast<float>(k / 64);
+    } else {
+        size_t bytes = lora_bytes + align_up(split_x_bf16_bytes(m, k));  // x limbs
+        if (splits > 1) bytes += align_up(static_cast<size_t>(splits) * m * n * sizeof(float));
+        plan.workspace_bytes = bytes;
+        const size_t rounds = (tiles * splits + dev.cu_count - 1) / dev.cu_count;
+        us = 9.0f + 0.75f * static_cast<float>(rounds) * static_cast<float>(per_split);
+        if (splits > 1)
+            us += 3.0f + 0.25f * static_cast<float>(splits) +  // a round of loads per four planes
+                  1.6e-6f * static_cast<float>(splits) * static_cast<float>(m) * static_cast<float>(n);
     }
-    size_t bytes = lora_bytes + align_up(split_x_bf16_bytes(m, k));  // x limbs
-    if (splits > 1) bytes += align_up(static_cast<size_t>(splits) * m * n * sizeof(float));
-    plan.workspace_bytes = bytes;
+    plan.contract_bytes = plan.workspace_bytes;
+    // Small and middling shapes leave most of either grid idle or its pipeline mostly filling; the digit
+    // kernel's 8-row tiles and single launch win there (us per call, limb GEMM -> digits: 128 x 64 -> 320
+    // 11.9 -> 3.4, 128 x 1024 -> 1024 19.4 -> 5.8, 64 x 4096 -> 4096 47.8 -> 18.5, 77 x 2880 -> 7001 38.3 -> 37.0;
+    // 256 x 4096 -> 2048, estimated 29 against 33, is 30 against 32.7).
+    if (digits.us < us) {
+        plan.kind = Q4Plan::kDigits;
+        plan.splits = 1;
+        plan.tiles = digits.tiles;
+        plan.workspace_bytes = lora_bytes;
+    }
     return plan;
 }
 
@@ -959,7 +971,7 @@ hipError_t launch_q4gemm(const Q4Plan& plan, const DeviceInfo& dev, const float*
                          float lora_scale, void* workspace, hipStream_t stream) {
     if (plan.kind == Q4Plan::kGemv) return launch_gemv(dev, x, w_packed, w_scales, y, m, n, k, stream);
     if (plan.kind == Q4Plan::kDigits)
-        return launch_q4gemm_small(dev, x, w_packed, w_scales, y, m, n, k, la, lb, rank, lora_scale, plan.t_splits,
+        return launch_q4gemm_small(dev, x, w_packed, w_scales, y, m, n, k, la, lb, rank, lora_scale, plan.t_splits, plan.tiles,
                                    workspace, stream);
     if (plan.kind == Q4Plan::kMid) {
         uint16_t* xs = static_cast<uint16_t*>(workspace);

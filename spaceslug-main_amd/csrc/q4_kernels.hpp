@@ -33,14 +33,18 @@ constexpr bool gemv_takes(uint32_t m, uint32_t k) {
 
 // Launch shape chosen by plan_q4gemm for one call.
 struct Q4Plan {
-    // kGemv: decode GEMV (gemv_takes, no LoRA); kDigits: every other call up to 32 rows,
-    // exact integer group sums on the int8 matrix cores (q4_small.hip); kWide: m > 32; kMid:
-    // m > 32 without LoRA whose 128 x 128 grid would need a K-split while its 64 x 64 grid fits
-    // the CUs once (k % 64 == 0, k <= 4096).
+    // kGemv: decode GEMV (gemv_takes, no LoRA); kDigits: every other call up to 32 rows, and taller
+    // ones whose estimate is the lowest, exact integer group sums on the int8 matrix cores
+    // (q4_small.hip); kWide: m > 32; kMid: m > 32 without LoRA whose 128 x 128 grid would need a
+    // K-split while its 64 x 64 grid fits the CUs once (k % 64 == 0, k <= 4096).
     enum Kind { kGemv, kDigits, kWide, kMid } kind;
     int splits;              // K-splits of the MFMA kernel (1 = write y directly)
     size_t workspace_bytes;  // device scratch the call needs (split partials, LoRA T partials and T, x limbs)
     int t_splits;            // K-splits of the LoRA pre-pass T = x * lora_a (0 without LoRA)
+    int tiles;               // kDigits: column tiles per workgroup, or 0 for q4_gemm_small_kernel
+    // Scratch by which the entry points accept or refuse a call (under stream capture, and against the
+    // fixed scratch): above 32 rows that of the limb GEMMs, whichever kernel runs.
+    size_t contract_bytes;
 };
 
 struct DeviceInfo {
@@ -63,11 +67,21 @@ hipError_t launch_q4gemm(const Q4Plan& plan, const DeviceInfo& dev, const float*
                          uint32_t n, uint32_t k, const float* la, const float* lb, uint32_t rank,
                          float lora_scale, void* workspace, hipStream_t stream);
 
-// Small-batch GEMM (kDigits, q4_small.hip): one launch, plus a preparation launch for the LoRA T
-// partials; `workspace` holds t_splits * m * rank floats of them (unused without LoRA).
+// Digit GEMMs (kDigits, q4_small.hip): one launch, plus a preparation launch for the LoRA T
+// partials; `workspace` holds t_splits * m * rank floats of them (unused without LoRA). `tiles` is the
+// plan's.
 hipError_t launch_q4gemm_small(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
                                float* y, uint32_t m, uint32_t n, uint32_t k, const float* la, const float* lb,
-                               uint32_t rank, float lora_scale, int t_splits, void* workspace, hipStream_t stream);
+                               uint32_t rank, float lora_scale, int t_splits, int tiles, void* workspace,
+                               hipStream_t stream);
+
+// Column tiles per workgroup of q4_gemm_tiles_kernel for (m, n, k), 0 where q4_gemm_small_kernel is the
+// better one, and the call's estimated time in microseconds.
+struct DigitTiles {
+    int tiles;
+    float us;
+};
+DigitTiles plan_digit_tiles(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k);
 
 // Bytes of the wide int4 GEMM's x limbs for x (fp32, m x k, k % 32 == 0): three exact bf16 limbs
 // per value in 16-row blocks (rows padded with zeros to a multiple of 16), written by the

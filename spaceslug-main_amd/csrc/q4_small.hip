@@ -1,6 +1,7 @@
-// Exact small-batch int4 GEMM: M <= 32 rows (and one row with K > 32768), any K % 32 == 0.
+// Exact int4 GEMMs on digits of x: every call up to 32 rows that the decode GEMV does not take, and
+// taller ones whose grids are too small for the limb GEMMs (plan_q4gemm); any K % 32 == 0.
 //
-// Replaces q4gemm.comp:61-175 for decode-sized batches. Every 32-value group sum
+// Replaces q4gemm.comp:61-175 for decode-sized batches and small shapes. Every 32-value group sum
 // sum_k x[m][k] * v[k][n] is formed exactly, in integers, on the int8 matrix cores, in one
 // launch with no device memory beyond the arguments (a LoRA call adds the T = x * la
 // partials of a preparation launch):
@@ -17,7 +18,8 @@
 //     + (S_0 + 256 S_1) is exact in double (|C| < 2^44) and y += C * s * 2^(e - 34) rounds
 //     once per group in double. No fp32 rounding touches a group sum, so the error does not
 //     grow with K the way an fp32 group sum's does.
-// Work mapping: a workgroup owns 8 rows x 32 columns (one MFMA tile; lane l of the result
+// q4_gemm_tiles_kernel, at its definition, shares one recoding among several column tiles.
+// Work mapping of q4_gemm_small_kernel: a workgroup owns 8 rows x 32 columns (one MFMA tile; lane l of the result
 // holds column l % 32, rows 2i + l / 32 for i < 4) and its wavefronts split K; their float64
 // accumulators are summed through LDS in wavefront order (deterministic). Per wavefront, x,
 // packed weights and scales reach LDS by buffer loads to LDS in chunks of 4 groups, three
@@ -26,6 +28,9 @@
 // Rows holding an infinity or a NaN are flagged while recoding and their outputs formed in
 // IEEE double arithmetic over the non-finite terms, which is the double reference's result
 // for such rows (test_q4gemm.cpp:102-119).
+#include <algorithm>
+#include <cfloat>
+#include <cmath>
 #include <type_traits>
 
 #include "q4_device.hpp"
@@ -85,6 +90,30 @@ __device__ __forceinline__ void copy_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_
             : "=&s"(saved)
             : "v"(voffset), "s"(rsrc), "s"(soffset), "s"(l)
             : "memory");
+}
+
+// Four such copies of B0 .. B3 bytes per lane to l, l + o1, l + o2 and l + o3 (the first two through r0, the others
+// through r1; lane offsets only). M0 is left at the last address.
+template <int B0, int B1, int B2, int B3>
+__device__ __forceinline__ void copy4_to_lds(__amdgpu_buffer_rsrc_t r0, __amdgpu_buffer_rsrc_t r1, uint32_t v0, uint32_t v1,
+                                             uint32_t v2, uint32_t v3, uint32_t l, uint32_t o1, uint32_t o2, uint32_t o3) {
+    const uint32_t l1 = l + o1, l2 = l + o2, l3 = l + o3;
+    if constexpr (B2 == 16)
+        asm volatile(
+            "s_mov_b32 m0, %6\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds\n\t"
+            "s_mov_b32 m0, %7\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
+            "s_mov_b32 m0, %8\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %5, 0 offen lds\n\t"
+            "s_mov_b32 m0, %9\n\ts_nop 0\n\tbuffer_load_dwordx4 %3, %5, 0 offen lds"
+            ::"v"(v0), "v"(v1), "v"(v2), "v"(v3), "s"(r0), "s"(r1), "s"(l), "s"(l1), "s"(l2), "s"(l3)
+            : "memory", "m0");
+    else
+        asm volatile(
+            "s_mov_b32 m0, %6\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds\n\t"
+            "s_mov_b32 m0, %7\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %4, 0 offen lds\n\t"
+            "s_mov_b32 m0, %8\n\ts_nop 0\n\tbuffer_load_dword %2, %5, 0 offen lds\n\t"
+            "s_mov_b32 m0, %9\n\ts_nop 0\n\tbuffer_load_dword %3, %5, 0 offen lds"
+            ::"v"(v0), "v"(v1), "v"(v2), "v"(v3), "s"(r0), "s"(r1), "s"(l), "s"(l1), "s"(l2), "s"(l3)
+            : "memory", "m0");
 }
 
 // Byte selectors of a 4 x 4 byte transpose whose outputs come in the order s ^ r.
@@ -162,7 +191,7 @@ __device__ float ieee_row_value(const float* x, const uint32_t* wq, const float*
 // NI: output register pairs per lane in use (rows 2 i + h, i < NI): 1 for M <= 2, 2 for M <= 4,
 // else 4. W: wavefronts per workgroup, splitting K. Every variant keeps four wavefronts per SIMD
 // resident (at most 128 VGPRs and 40 KiB of LDS per wavefront), which hides the recoding's
-// dependent chains.
+// dependent chains. Taken for short K and for some grids of one tile per CU (plan_digit_tiles).
 template <int NI, int W>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void q4_gemm_small_kernel(const float* x, const uint32_t* wq, const float* ws,
                                                                float* __restrict__ y, int M, int N, int K, int RB,
@@ -443,21 +472,329 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
     }
 }
 
-template <int NI, int W>
-hipError_t launch_small_gemm(const float* x, const uint8_t* w_packed, const float* w_scales, float* y, int m, int n,
-                             int k, int RB, int tiles_n, const float* tpart, int t_splits, const float* lb, int rank,
-                             float lscale, hipStream_t stream) {
-    hipLaunchKernelGGL((q4_gemm_small_kernel<NI, W>), dim3(static_cast<unsigned>(RB * tiles_n)), dim3(64 * W), 0,
-                       stream, x, reinterpret_cast<const uint32_t*>(w_packed), w_scales, y, m, n, k, RB, tiles_n,
-                       tpart, t_splits, lb, rank, lscale);
-    return hipGetLastError();
+// The same exact products for tiles that share their recoding: a workgroup owns 8 rows x 32 CT
+// columns. Issue-bound: per group a wavefront spends ~36 VALU instructions on recoding 8 rows and
+// ~35 on each tile of 32 columns (28 of them the float64 fold), so with one tile per recoding
+// (q4_gemm_small_kernel) more than half of the work is repeated by every column tile. CT is chosen
+// so that the grid fits the CUs once where it can (launch_q4gemm_small). Eight wavefronts (two per SIMD)
+// deal K among themselves in chunks of four groups:
+//   - x of a chunk (4 KiB) and, per column tile, its packed weights (2 KiB, 64 contiguous bytes per
+//     column) and scales come by copies to LDS; the weights kTileRing tiles ahead, x one chunk
+//     ahead. Nothing else is loaded from memory in the loop, so the waits are exact counts; copies
+//     past the last chunk read nothing and keep the counts;
+//   - lane (row r = lane / 8, octet o = lane % 8) recodes the eight values of word o % 4 of group
+//     o / 4 for two pairs of groups: two 16-byte reads, the group maximum over its quad of lanes, and
+//     two byte transposes (even and odd nibble positions) written as 8-byte pieces of the four A
+//     lanes (row, digit, half). 16-byte units of odd rows sit swapped, so reads meet distinct banks;
+//   - the chunk's digits and exponents then stay in registers for all CT tiles; per tile a lane
+//     reads its 8 bytes of each group (slot g ^ (column / 4 % 4) of the column's 64 bytes: 16
+//     columns meet all banks) and four scales one tile ahead of their use.
+constexpr int kTileGroups = 4;                                   // groups per chunk
+constexpr int kTileRing = 4;                                     // weight tiles in flight per wavefront
+constexpr int kTileWaves = 8;
+constexpr int kTileXBytes = kTileGroups * kDigitRows * 128;      // x of a chunk, then its digits
+constexpr int kTileWBytes = kDigitCols * kTileGroups * 16;       // packed weights of a tile's chunk
+constexpr int kTileSlot = kTileWBytes + kDigitCols * kTileGroups * 4;
+constexpr int kTileWaveBytes = 2 * kTileXBytes + kTileRing * kTileSlot + kTileGroups * kDigitRows * 4;
+
+template <int CT, int NI>
+__global__ __launch_bounds__(64 * kTileWaves) void q4_gemm_tiles_kernel(const float* x, const uint32_t* wq, const float* ws,
+                                                                       float* __restrict__ y, int M, int N, int K, int RB,
+                                                                       int blocks_n, const float* __restrict__ tpart,
+                                                                       int t_splits, const float* __restrict__ lb, int R,
+                                                                       float lscale) {
+    constexpr int W = kTileWaves;
+    __shared__ __align__(16) unsigned char lds[W * kTileWaveBytes];
+    __shared__ int rowmask;
+    static_assert(W * CT * NI * 64 * 8 + kDigitRows * kMaxLoraRank * 4 <= W * kTileWaveBytes, "epilogue partials and T fit");
+    const int lane = static_cast<int>(threadIdx.x) & 63;
+    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int c = lane & 31, h = lane >> 5;
+    const int G = K >> 5;
+    // Row blocks fastest, in runs per XCD (workgroup i runs on XCD i % 8): the row blocks that share
+    // columns share their weights in one L2.
+    int lin = static_cast<int>(blockIdx.x);
+    const int total = RB * blocks_n;
+    const int run = (total + 7) >> 3;
+    lin = (lin & 7) * run + (lin >> 3);
+    if (lin >= total) return;  // the grid is 8 * run
+    const int m0 = (lin % RB) * kDigitRows;
+    const int n0 = (lin / RB) * (kDigitCols * CT);
+    if (threadIdx.x == 0) rowmask = 0;
+    __syncthreads();
+
+    const int nct = (G + kTileGroups - 1) / kTileGroups;
+    const int nchunks = nct > w ? (nct - w + W - 1) / W : 0;
+    auto chunk_group = [&](int j) { return (w + j * W) * kTileGroups; };
+
+    unsigned char* const wl = lds + w * kTileWaveBytes;
+    unsigned char* const ring = wl + 2 * kTileXBytes;
+    int* const xexp = reinterpret_cast<int*>(ring + kTileRing * kTileSlot);
+
+    // Copy sources: x rows 4 i + lane / 16, unit (lane % 16) ^ (row & 1) of a pair of groups' 256
+    // bytes; weights of column 16 i + lane / 4, group (lane % 4) ^ (column / 4 % 4); scales the same
+    // without the swap. A copy's whole offset is in its lanes (the range check then needs no scalar
+    // offset), so reads past the end (rows past M, columns past N, chunks past the last) return zeros.
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(x + static_cast<size_t>(m0) * K, static_cast<size_t>(M - m0) * K * 4);
+    const __amdgpu_buffer_rsrc_t rw =
+        make_rsrc(wq + static_cast<size_t>(n0) * G * 4, static_cast<size_t>(N - n0) * G * 16);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(ws + static_cast<size_t>(n0) * G, static_cast<size_t>(N - n0) * G * 4);
+    const uint32_t vx = static_cast<uint32_t>((lane >> 4) * K * 4 + ((lane & 15) ^ ((lane >> 4) & 1)) * 16);
+    const uint32_t vw = static_cast<uint32_t>(((lane >> 2) * G + ((lane & 3) ^ ((lane >> 4) & 3))) * 16);
+    const uint32_t vs = static_cast<uint32_t>(((lane >> 2) * G + (lane & 3)) * 4);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)(lds_ptr)wl);
+    constexpr uint32_t kPast = 0x7FFFFFFFu;
+    constexpr int kXCopies = 4, kWCopies = 4;
+    auto issue_x = [&](int j, int buf) {
+        const uint32_t so = j < nchunks ? static_cast<uint32_t>(chunk_group(j) * 128) : kPast;
+        const uint32_t row4 = j < nchunks ? static_cast<uint32_t>(16 * K) : 0u;
+        copy4_to_lds<16, 16, 16, 16>(rx, rx, vx + so, vx + (so + row4), vx + (so + (j < nchunks ? 256u : 0u)),
+                                     vx + (so + row4 + (j < nchunks ? 256u : 0u)), lds0 + buf * kTileXBytes, 1024, 2048, 3072);
+    };
+    // The tile of column group offset `off` (in groups from the workgroup's first column) into ring slot `slot`.
+    auto issue_w = [&](uint32_t off, int slot) {
+        const uint32_t half = off == kPast ? 0u : static_cast<uint32_t>(16 * G);
+        const uint32_t b16 = off == kPast ? kPast : off * 16u, b4 = off == kPast ? kPast : off * 4u;
+        copy4_to_lds<16, 16, 4, 4>(rw, rs, vw + b16, vw + (b16 + half * 16u), vs + b4, vs + (b4 + half * 4u),
+                                   lds0 + 2 * kTileXBytes + slot * kTileSlot, 1024, 2048, 2304);
+    };
+
+    const int rr = lane >> 3, oct = lane & 7, rg = oct >> 2, rh = (oct >> 1) & 1;
+    const int xoff0 = rr * 256 + ((2 * oct) ^ (rr & 1)) * 16, xoff1 = rr * 256 + ((2 * oct + 1) ^ (rr & 1)) * 16;
+    const int dr = 2 * rh + (rr >> 2);  // digit order, so that a write instruction spreads over the banks
+    const TransposeSel tsel(dr);
+    int wofs[4];
+#pragma unroll
+    for (int sl = 0; sl < 4; ++sl) wofs[sl] = rg * 1024 + (32 * rh + 4 * rr + (sl ^ dr)) * 16 + 8 * (oct & 1);
+    uint32_t mbrun = 0;
+    // Recodes the chunk at group cb in place: digits of group g at 1024 g, exponents to xexp.
+    auto recode = [&](unsigned char* xb, int cb) {
+        f32x4 v[2][2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            v[p][0] = *reinterpret_cast<const f32x4*>(xb + p * 2048 + xoff0);
+            v[p][1] = *reinterpret_cast<const f32x4*>(xb + p * 2048 + xoff1);
+        }
+        if (cb + kTileGroups > G) {  // uniform: groups past K hold the next row's values
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                if (cb + 2 * p + rg >= G) v[p][0] = v[p][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            uint32_t mb = 0;
+#pragma unroll
+            for (int i = 0; i < 8; i += 2)
+                mb = max(mb, max(__float_as_uint(v[p][i >> 2][i & 3]) & 0x7FFFFFFFu,
+                                 __float_as_uint(v[p][i >> 2][(i & 3) + 1]) & 0x7FFFFFFFu));
+            mb = max(mb, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(mb), 0xB1, 0xF, 0xF, false)));
+            mb = max(mb, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(mb), 0x4E, 0xF, 0xF, false)));
+            mbrun = max(mbrun, mb);
+            const int e = __builtin_amdgcn_frexp_expf(__uint_as_float(mb));  // max < 2^e (0: all-zero group)
+            const int sh = kDigitFracBits - e;
+            uint32_t z[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                z[i] = (static_cast<uint32_t>(round_half_up(ldexpf(v[p][i >> 2][i & 3], sh))) + kDigitBias) ^ kDigitBias;
+            uint32_t even[4], odd[4];  // [sl]: digit sl ^ dr of the values at even and odd positions
+            transpose_bytes(z[0], z[2], z[4], z[6], tsel, even);
+            transpose_bytes(z[1], z[3], z[5], z[7], tsel, odd);
+#pragma unroll
+            for (int sl = 0; sl < 4; ++sl)
+                *reinterpret_cast<uint2*>(xb + p * 2048 + wofs[sl]) = uint2{even[sl], odd[sl]};
+            xexp[(2 * p + rg) * kDigitRows + exp_slot(rr)] = e - 34;  // the group's four lanes store the same value
+        }
+    };
+
+    struct Words {
+        uint2 w[kTileGroups];
+        f32x4 s;
+    };
+    const int woff = (c >> 4) * 1024 + (c & 15) * 64 + 8 * h;
+    const unsigned char* wsrc[kTileGroups];
+#pragma unroll
+    for (int g = 0; g < kTileGroups; ++g) wsrc[g] = ring + woff + (g ^ ((c >> 2) & 3)) * 16;
+    const unsigned char* const ssrc = ring + kTileWBytes + c * 16;
+    auto read_words = [&](Words& d, int slot) {
+#pragma unroll
+        for (int g = 0; g < kTileGroups; ++g) d.w[g] = *reinterpret_cast<const uint2*>(wsrc[g] + slot * kTileSlot);
+        d.s = *reinterpret_cast<const f32x4*>(ssrc + slot * kTileSlot);
+    };
+
+    double acc[CT][NI];
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) acc[t][i] = 0.0;
+    i32x4 dig[kTileGroups], ex[kTileGroups];
+    auto product = [&](int g, const Words& d) {
+        const i32x16 zero = {};
+        return __builtin_amdgcn_mfma_i32_32x32x32_i8(dig[g], weights_i8x16(d.w[g].x, d.w[g].y), zero, 0, 0, 0);
+    };
+    auto fold = [&](double (&a)[NI], const i32x16& r, float sf, const i32x4& e4) {
+        const double sd = static_cast<double>(sf);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int lo = r[4 * i] + (r[4 * i + 1] << 8);
+            const int hi = r[4 * i + 2] + (r[4 * i + 3] << 8);
+            const double cg = fma(static_cast<double>(hi), 65536.0, static_cast<double>(lo));
+            a[i] = fma(cg, ldexp(sd, e4[i]), a[i]);
+        }
+    };
+
+    // Step i = (chunk j, tile t) works on words read during step i - 1, while the ring holds the tiles
+    // of steps i + 1 .. i + 4. kUnroll chunks are a multiple of four steps and of two chunks, so that ring
+    // slots and x buffers are constants. Tile t of chunk j starts 32 t G groups and the chunk's
+    // position from the first column.
+    constexpr int kUnroll = CT % 2 ? 4 : 2;
+    static_assert(kUnroll * CT % kTileRing == 0 && kTileRing == 4, "ring slots are constants");
+    Words words[2];
+    // Issues the tile of step i + 4, i the step u of the chunks from chunk j on.
+    auto issue_ahead = [&](int j, auto uc) {
+        constexpr int u = decltype(uc)::value + kTileRing;
+        const int ja = j + u / CT;
+        issue_w(ja < nchunks ? static_cast<uint32_t>(chunk_group(ja) + (u % CT) * kDigitCols * G) : kPast, u % kTileRing);
+    };
+    if (nchunks > 0) {
+        issue_x(0, 0);
+        static_for<kTileRing>([&](auto uc) { issue_ahead(0, std::integral_constant<int, decltype(uc)::value - kTileRing>{}); });
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kTileRing - 1) * kWCopies) : "memory");
+        read_words(words[0], 0);
+    }
+    auto run_chunk = [&](int j, auto pc) {
+        constexpr int pass = decltype(pc)::value;  // chunk j is the pass-th of an unrolled body
+        const int cb = chunk_group(j);
+        static_for<CT>([&](auto tc) {
+            constexpr int t = decltype(tc)::value;
+            constexpr int u = pass * CT + t;
+            Words& cur = words[u & 1];
+            Words& nxt = words[(u + 1) & 1];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this step's words are in registers
+            issue_ahead(j - pass, std::integral_constant<int, u>{});
+            if constexpr (t == 0) {
+                // x of this chunk: behind it only the tiles issued since
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CT * kWCopies) : "memory");
+                unsigned char* xb = wl + (pass & 1) * kTileXBytes;
+                recode(xb, cb);
+                issue_x(j + 1, (pass & 1) ^ 1);
+#pragma unroll
+                for (int g = 0; g < kTileGroups; ++g) {
+                    dig[g] = *reinterpret_cast<const i32x4*>(xb + g * 1024 + lane * 16);
+                    ex[g] = *reinterpret_cast<const i32x4*>(xexp + g * kDigitRows + h * 4);
+                }
+            }
+            // the next step's tile: behind it three tiles and, issued in the last three steps, the next x
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kTileRing - 1) * kWCopies + (t < kTileRing ? kXCopies : 0)) : "memory");
+            read_words(nxt, (u + 1) % kTileRing);
+            f32x4 s = cur.s;  // the scales of groups past K belong to the next column
+#pragma unroll
+            for (int g = 1; g < kTileGroups; ++g) s[g] = cb + g < G ? s[g] : 0.0f;
+            i32x16 p0 = product(0, cur);
+            i32x16 p1 = product(1, cur);
+            __builtin_amdgcn_sched_barrier(0);
+            fold(acc[t], p0, s[0], ex[0]);
+            p0 = product(2, cur);
+            __builtin_amdgcn_sched_barrier(0);
+            fold(acc[t], p1, s[1], ex[1]);
+            p1 = product(3, cur);
+            __builtin_amdgcn_sched_barrier(0);
+            fold(acc[t], p0, s[2], ex[2]);
+            fold(acc[t], p1, s[3], ex[3]);
+            // pins the fold here: sunk to the next use of the sums it would keep four products alive
+#pragma unroll
+            for (int i = 0; i < NI; ++i) asm volatile("" : "+v"(acc[t][i]));
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    for (int j0 = 0; j0 < nchunks; j0 += kUnroll)
+        static_for<kUnroll>([&](auto pc) {
+            if (j0 + decltype(pc)::value < nchunks) run_chunk(j0 + decltype(pc)::value, pc);  // uniform
+        });
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // copies past the last step still write LDS
+
+    if (mbrun >= 0x7F800000u) atomicOr(&rowmask, 1 << rr);  // rare: a row with an infinity or a NaN
+    __syncthreads();  // every wavefront's K range is done: its staging is free
+    double* red = reinterpret_cast<double*>(lds);  // [wavefront][tile][i][lane]
+    float* lora_t_s = reinterpret_cast<float*>(red + W * CT * NI * 64);  // [8 rows][R]
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) red[((w * CT + t) * NI + i) * 64 + lane] = acc[t][i];
+    if (lb != nullptr) {
+        for (int e0 = static_cast<int>(threadIdx.x); e0 < kDigitRows * R; e0 += 64 * W) {
+            float tv[1];
+            lora_t_values<1>(tpart, t_splits, M, R, 0, R, m0, e0, 64 * W, kDigitRows * R, tv);
+            lora_t_s[e0] = tv[0];
+        }
+    }
+    __syncthreads();
+    for (int e = static_cast<int>(threadIdx.x); e < kDigitRows * kDigitCols * CT; e += 64 * W) {
+        const int ml = e / (kDigitCols * CT), cc = e % (kDigitCols * CT);
+        const int m = m0 + ml, n = n0 + cc;
+        const int i = ml >> 1;
+        if (m >= M || n >= N) continue;
+        double s = 0.0;
+        if (i < NI) {
+#pragma unroll
+            for (int v = 0; v < W; ++v) s += red[((v * CT + (cc >> 5)) * NI + i) * 64 + (cc & 31) + 32 * (ml & 1)];
+        }
+        if ((rowmask >> ml) & 1) s = ieee_row_value(x, wq, ws, m, n, K);
+        if (lb != nullptr) {
+            double tb = 0.0;
+#pragma unroll 8
+            for (int r = 0; r < R; ++r)
+                tb = fma(static_cast<double>(lora_t_s[ml * R + r]), static_cast<double>(lb[static_cast<size_t>(r) * N + n]), tb);
+            s = fma(static_cast<double>(lscale), tb, s);
+        }
+        y[static_cast<size_t>(m) * N + n] = static_cast<float>(s);
+    }
 }
 
 }  // namespace
 
+// Estimate fitted to the measured calls of 3 to 512 rows: per round of workgroups on the CUs and unit of
+// (CT + 2) tiles (recoding costs as much as about two tiles), 0.61 us for each chunk of a wavefront plus
+// 0.3; below one chunk per wavefront the fixed part of a workgroup, 0.6. CT is the one with the
+// lowest product, a single round where that does not lengthen it: 27 x 4096 -> 11001 takes 24.8 us at
+// CT = 6 (232 workgroups), 34.2 at 4 and 29.0 at 8; 39.2 on q4_gemm_small_kernel.
+DigitTiles plan_digit_tiles(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k) {
+    if (k > (1u << 22)) return {0, FLT_MAX};  // beyond 32-bit offsets of 256 columns
+    const size_t rb = (m + kDigitRows - 1) / kDigitRows, tiles_n = (n + kDigitCols - 1) / kDigitCols;
+    const size_t cus = static_cast<size_t>(dev.cu_count);
+    size_t best = 0;
+    int tiles = 0;
+    for (int ct : {1, 2, 3, 4, 5, 6, 8}) {
+        const size_t rounds = (rb * ((tiles_n + ct - 1) / ct) + cus - 1) / cus;
+        const size_t units = rounds * static_cast<size_t>(ct + 2);
+        if (tiles == 0 || units < best) {
+            best = units;
+            tiles = ct;
+        }
+    }
+    const float chunks = static_cast<float>((k / kGroup + kTileGroups - 1) / kTileGroups) / kTileWaves;
+    const float us = 2.8f + static_cast<float>(best) * std::max(0.6f, 0.3f + 0.61f * (chunks < 1.0f ? chunks : std::ceil(chunks)));
+    // q4_gemm_small_kernel keeps a short K, whose few chunks its smaller workgroups spread over more
+    // CUs (32 x 192 -> 10000 5.2 against 6.2 us; at K = 512 7.5 against 6.6).
+    if (k < 512) return {0, 3.2f + static_cast<float>(rb * tiles_n) * (1.0e-3f + 3.2e-6f * static_cast<float>(k))};
+    // With one tile per workgroup it also keeps
+    //   - K below 3072, unless the chunks fill whole rounds of the wavefronts: its shorter chunks divide
+    //     more evenly (16 -> 4000 columns: K = 1024 4.6 against 4.8 us, 2688 7.7 against 7.8; but 2048 6.8
+    //     against 6.5, 3072 8.5 against 7.9, 4096 10.5 against 9.3);
+    //   - up to four rows below K = 7168, where half or more of the fold falls away and recoding is what
+    //     counts (3 -> 2000 columns: K = 2688 6.4 against 7.1 us, 5824 10.3 against 10.9, 7488 12.9 against 12.7);
+    //   - one row block with a tile on nearly every CU and K up to 8192: its deeper copies hide the
+    //     weights' latency better (8 x 4096 -> 8192 columns 10.6 against 11.0 us, -> 7000 10.3 against 9.8).
+    const bool whole_rounds = k % (kTileWaves * kTileGroups * kGroup) == 0 && k >= 2048;
+    if (tiles == 1 && ((k < 3072 && !whole_rounds) || (m <= 4 && k < 7168) ||
+                       (rb == 1 && 8 * tiles_n > 7 * cus && k <= 8192)))
+        tiles = 0;
+    return {tiles, us};
+}
+
 hipError_t launch_q4gemm_small(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
                                float* y, uint32_t m, uint32_t n, uint32_t k, const float* la, const float* lb,
-                               uint32_t rank, float lora_scale, int t_splits, void* workspace, hipStream_t stream) {
+                               uint32_t rank, float lora_scale, int t_splits, int tiles, void* workspace,
+                               hipStream_t stream) {
     const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
     const int RB = (M + kDigitRows - 1) / kDigitRows;
     const int R = static_cast<int>(rank);
@@ -471,24 +808,46 @@ hipError_t launch_q4gemm_small(const DeviceInfo& dev, const float* x, const uint
         if (pe != hipSuccess) return pe;
     }
     const int tiles_n = (N + kDigitCols - 1) / kDigitCols;
-    // Wavefronts per workgroup: 16 per CU in total, whether one, two or four workgroups share a CU.
-    const int total = RB * tiles_n;
-    const int W = total <= dev.cu_count ? 16 : total <= 2 * dev.cu_count ? 8 : 4;
-    const int NI = M <= 2 ? 1 : M <= 4 ? 2 : 4;
     const float* lbp = rank ? lb : nullptr;
-    auto go = [&](auto ni, auto wv) {
-        return launch_small_gemm<decltype(ni)::value, decltype(wv)::value>(x, w_packed, w_scales, y, M, N, K, RB,
-                                                                           tiles_n, tpart, t_splits, lbp, R,
-                                                                           lora_scale, stream);
+    const uint32_t* wq = reinterpret_cast<const uint32_t*>(w_packed);
+    auto go = [&](auto ct, auto ni) {
+        constexpr int CT = decltype(ct)::value, NI = decltype(ni)::value;
+        if constexpr (CT == 0) {
+            // 16 wavefronts per CU in total, whether one, two or four workgroups share it
+            const size_t total = static_cast<size_t>(RB) * tiles_n;
+            auto small = [&](auto wv) {
+                constexpr int W = decltype(wv)::value;
+                hipLaunchKernelGGL((q4_gemm_small_kernel<NI, W>), dim3(static_cast<unsigned>(total)), dim3(64 * W), 0, stream, x,
+                                   wq, w_scales, y, M, N, K, RB, tiles_n, tpart, t_splits, lbp, R, lora_scale);
+            };
+            if (total <= static_cast<size_t>(dev.cu_count)) small(std::integral_constant<int, 16>{});
+            else if (total <= 2 * static_cast<size_t>(dev.cu_count)) small(std::integral_constant<int, 8>{});
+            else small(std::integral_constant<int, 4>{});
+        } else {
+            const int blocks_n = (tiles_n + CT - 1) / CT;
+            const unsigned grid = static_cast<unsigned>((RB * static_cast<size_t>(blocks_n) + 7) / 8 * 8);
+            hipLaunchKernelGGL((q4_gemm_tiles_kernel<CT, NI>), dim3(grid), dim3(64 * kTileWaves), 0, stream, x, wq, w_scales, y,
+                               M, N, K, RB, blocks_n, tpart, t_splits, lbp, R, lora_scale);
+        }
+        return hipGetLastError();
     };
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    using I4 = std::integral_constant<int, 4>;
-    using W16 = std::integral_constant<int, 16>;
-    using W8 = std::integral_constant<int, 8>;
-    if (NI == 1) return W == 16 ? go(I1{}, W16{}) : W == 8 ? go(I1{}, W8{}) : go(I1{}, I4{});
-    if (NI == 2) return W == 16 ? go(I2{}, W16{}) : W == 8 ? go(I2{}, W8{}) : go(I2{}, I4{});
-    return W == 16 ? go(I4{}, W16{}) : W == 8 ? go(I4{}, W8{}) : go(I4{}, I4{});
+    // Result register pairs in use (rows 2 i + h, i < NI).
+    auto by_rows = [&](auto ct) {
+        if (M <= 2) return go(ct, std::integral_constant<int, 1>{});
+        if (M <= 4) return go(ct, std::integral_constant<int, 2>{});
+        return go(ct, std::integral_constant<int, 4>{});
+    };
+    switch (tiles) {
+        case 0: return by_rows(std::integral_constant<int, 0>{});
+        case 1: return by_rows(std::integral_constant<int, 1>{});
+        case 2: return by_rows(std::integral_constant<int, 2>{});
+        case 3: return by_rows(std::integral_constant<int, 3>{});
+        case 4: return by_rows(std::integral_constant<int, 4>{});
+        case 5: return by_rows(std::integral_constant<int, 5>{});
+        case 6: return by_rows(std::integral_constant<int, 6>{});
+        case 8: return by_rows(std::integral_constant<int, 8>{});
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace spaceslug

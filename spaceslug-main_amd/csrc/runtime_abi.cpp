@@ -276,15 +276,17 @@ int run_device(const float* dx, const uint8_t* dw, const float* ds, const float*
     DeviceState& dev = current_device();
     const spaceslug::Q4Plan plan = spaceslug::plan_q4gemm(dev.info, m, n, k, rank);
     const hipStream_t st = static_cast<hipStream_t>(stream);
+    // A graph captured from this stream would keep the shared workspace's address, which a
+    // later, larger call frees: refuse before touching it. What is refused depends on the shape's
+    // contract (rows, rank), not on whether the kernel chosen for it happens to need the workspace.
+    if (plan.contract_bytes != 0)
+        if (const int rc = refuse_capture(st, "q4gemm")) return rc;
     if (plan.workspace_bytes == 0) {
         check(spaceslug::launch_q4gemm(plan, dev.info, dx, dw, ds, dy, m, n, k, dla, dlb, rank, lora_scale, nullptr,
                                        st),
               "q4gemm launch");
         return ok();
     }
-    // A graph captured from this stream would keep the shared workspace's address, which a
-    // later, larger call frees: refuse before touching it.
-    if (const int rc = refuse_capture(st, "q4gemm")) return rc;
     // Calls that use the shared workspace are ordered across streams: a call on a
     // stream other than the previous user's waits (on the GPU) for that user's end.
     std::lock_guard<std::mutex> lock(g_device_mutex);
@@ -490,9 +492,9 @@ int spaceslug_q4gemm_device_noalloc(const float* d_x, const uint8_t* d_w_packed,
     try {
         DeviceState& dev = current_device();
         const spaceslug::Q4Plan plan = spaceslug::plan_q4gemm(dev.info, m, n, k, 0);
-        if (plan.workspace_bytes > kNoAllocScratchBytes)
-            return fail(SPACESLUG_ERR_INVALID, "spaceslug_q4gemm_device_noalloc: this shape needs " +
-                                                   std::to_string(plan.workspace_bytes) +
+        if (plan.contract_bytes > kNoAllocScratchBytes)  // whichever kernel would run
+            return fail(SPACESLUG_ERR_INVALID, "spaceslug_q4gemm_device_noalloc: this shape is held to " +
+                                                   std::to_string(plan.contract_bytes) +
                                                    " bytes of scratch, more than the fixed " +
                                                    std::to_string(kNoAllocScratchBytes));
         // every byte of scratch a call reads was written earlier in that call: nothing to clear
