@@ -214,3 +214,28 @@ def test_gpu_quantize_file_cli_round_trip(session, oracle, gpu, tmp_path):
     p_o, s_o = oracle.q4_quantize(w)
     assert np.array_equal(t.packed, p_o) and same(t.scales, s_o)
     assert q4file.main(["info", str(tmp_path / "w.ssq4")]) == 0
+
+
+# The kernel's forms (64- and 128-column blocks of 2, 4 and 8 groups, the matrix read through or past the
+# caches) at ragged column and group counts, on values that sit on and one ulp beside every rounding tie
+# and clamp, and on groups of extreme magnitude: bytes and scales equal the oracle's.
+@pytest.mark.gpu
+@pytest.mark.parametrize("k,n", [(32, 65), (224, 129), (288, 63), (3104, 2100), (64, 530000), (4128, 8200)])
+def test_gpu_quantizer_forms_and_ties(session, oracle, gpu, k, n):
+    print(f"[gpu-case] quantize ties k={k} n={n}", flush=True)
+    rng = np.random.default_rng(k + n)
+    rows = min(k, 96)
+    step = np.float32(2.0) ** rng.integers(-20, 20, n).astype(np.float32) * (1 + rng.random(n, dtype=np.float32))
+    w = rng.integers(-16, 17, (rows, n)).astype(np.float32) * (step / 2)    # halves of a step: ties and integers
+    toward = np.where(rng.integers(0, 3, (rows, n)) == 0, np.float32(np.inf), w)
+    w = np.nextafter(w, np.where(rng.integers(0, 3, (rows, n)) == 0, np.float32(-np.inf), toward))
+    w[::32] = 8 * step                                                      # the group's extreme: scale = -step
+    w = np.tile(w, (k // rows + 1, 1))[:k].copy()
+    w[0:32, 0] *= np.float32(1e-37) / step[0]                               # subnormal quotient range
+    if n > 70:
+        w[0:32, 64] = np.float32(3e38) * rng.uniform(-1, 1, 32).astype(np.float32)
+        w[0:32, 65] = np.float32(1e-45) * rng.integers(-9, 10, 32).astype(np.float32)
+    packed, scales = session.q4_quantize_values(w, n, k)
+    p_o, s_o = oracle.q4_quantize(w)
+    assert np.array_equal(packed, p_o)
+    assert same(scales, s_o)
