@@ -910,10 +910,19 @@ Q4Plan plan_q4gemm(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, ui
         lora_bytes += align_up(static_cast<size_t>(plan.t_splits) * m * rank * sizeof(float));  // T partials
     }
     const DigitTiles digits = plan_digit_tiles(dev, m, n, k);
-    if (m <= 32) {
+    auto take_digits = [&] {
         plan.kind = Q4Plan::kDigits;
+        plan.splits = 1;
         plan.tiles = digits.tiles;
-        plan.workspace_bytes = plan.contract_bytes = lora_bytes;  // the T partials of a LoRA call; none otherwise
+        plan.workspace_bytes = lora_bytes;  // the T partials of a LoRA call; none otherwise
+        if (rank > 0 && digits.tiles == 0 && digits_lora_in_kernel(dev, m, n, k, rank)) {
+            plan.t_splits = 0;
+            plan.workspace_bytes = 0;
+        }
+    };
+    if (m <= 32) {
+        plan.contract_bytes = lora_bytes;
+        take_digits();
         return plan;
     }
     plan.kind = Q4Plan::kWide;
@@ -956,12 +965,7 @@ Q4Plan plan_q4gemm(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, ui
     // kernel's 8-row tiles and single launch win there (us per call, limb GEMM -> digits: 128 x 64 -> 320
     // 11.9 -> 3.4, 128 x 1024 -> 1024 19.4 -> 5.8, 64 x 4096 -> 4096 47.8 -> 18.5, 77 x 2880 -> 7001 38.3 -> 37.0;
     // 256 x 4096 -> 2048, estimated 29 against 33, is 30 against 32.7).
-    if (digits.us < us) {
-        plan.kind = Q4Plan::kDigits;
-        plan.splits = 1;
-        plan.tiles = digits.tiles;
-        plan.workspace_bytes = lora_bytes;
-    }
+    if (digits.us < us) take_digits();
     return plan;
 }
 

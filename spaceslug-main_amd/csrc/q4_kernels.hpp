@@ -40,7 +40,7 @@ struct Q4Plan {
     enum Kind { kGemv, kDigits, kWide, kMid } kind;
     int splits;              // K-splits of the MFMA kernel (1 = write y directly)
     size_t workspace_bytes;  // device scratch the call needs (split partials, LoRA T partials and T, x limbs)
-    int t_splits;            // K-splits of the LoRA pre-pass T = x * lora_a (0 without LoRA)
+    int t_splits;            // K-splits of the LoRA pre-pass T = x * lora_a (0: none)
     int tiles;               // kDigits: column tiles per workgroup, or 0 for q4_gemm_small_kernel
     // Scratch by which the entry points accept or refuse a call (under stream capture, and against the
     // fixed scratch): above 32 rows that of the limb GEMMs, whichever kernel runs.
@@ -68,8 +68,8 @@ hipError_t launch_q4gemm(const Q4Plan& plan, const DeviceInfo& dev, const float*
                          float lora_scale, void* workspace, hipStream_t stream);
 
 // Digit GEMMs (kDigits, q4_small.hip): one launch, plus a preparation launch for the LoRA T
-// partials; `workspace` holds t_splits * m * rank floats of them (unused without LoRA). `tiles` is the
-// plan's.
+// partials; `workspace` holds t_splits * m * rank floats of them (unused without LoRA, and with
+// t_splits == 0, where the kernel computes T itself). `tiles` is the plan's.
 hipError_t launch_q4gemm_small(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
                                float* y, uint32_t m, uint32_t n, uint32_t k, const float* la, const float* lb,
                                uint32_t rank, float lora_scale, int t_splits, int tiles, void* workspace,
@@ -81,6 +81,7 @@ struct DigitTiles {
     int tiles;
     float us;
 };
+bool digits_lora_in_kernel(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, uint32_t rank);
 DigitTiles plan_digit_tiles(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k);
 
 // Bytes of the wide int4 GEMM's x limbs for x (fp32, m x k, k % 32 == 0): three exact bf16 limbs

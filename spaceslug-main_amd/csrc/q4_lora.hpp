@@ -47,6 +47,72 @@ __device__ __forceinline__ void lora_t_values(const float* __restrict__ tpart, i
     for (int v = 0; v < NV; ++v) out[v] = static_cast<float>(t[v]);
 }
 
+// T = x * la of a workgroup's own ROWS rows (from m0 on; rows past M - 1 repeat it), computed by its THREADS
+// threads for calls whose K * R is so small that a launch of its own would cost more
+// (lora_in_kernel): thread (slice, row, rank) takes every S-th run of four values of K in fp32, four
+// runs or, where the threads do not reach, up to kLoraRuns, all its loads issued before its first
+// product; the S slices are added in double, in order, and rounded once. Two steps around a
+// barrier: lora_rows_load leaves the slice sums in `part` (at most THREADS floats), lora_rows_sum returns
+// element threadIdx.x of T ([ROWS][R]).
+constexpr int kLoraRuns = 8;
+template <int ROWS, int THREADS>
+constexpr bool lora_in_kernel(uint32_t k, uint32_t rank) {
+    const uint32_t outs = ROWS * rank;
+    return rank > 0 && outs <= THREADS && k / 4 <= kLoraRuns * (THREADS / outs);
+}
+template <int THREADS>
+__device__ __forceinline__ int lora_slices(int K, int outs) {
+    return min(((K >> 2) + 3) >> 2, THREADS / outs);
+}
+template <int RUNS>
+__device__ __forceinline__ float lora_rows_slice(const float* __restrict__ xr, const float* __restrict__ lr, int R,
+                                                 int slice, int slices, int runs) {
+    f32x4 xv[RUNS], lv[RUNS];
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i) {
+        const int run = min(slice + i * slices, runs - 1);  // past the last: in bounds, dropped below
+        xv[i] = *reinterpret_cast<const f32x4*>(xr + 4 * run);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) lv[i][t] = lr[static_cast<size_t>(4 * run + t) * R];
+    }
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float p = fmaf(xv[i][t], lv[i][t], sum);
+            sum = slice + i * slices < runs ? p : sum;
+        }
+    return sum;
+}
+template <int ROWS, int THREADS>
+__device__ __forceinline__ void lora_rows_load(const float* __restrict__ x, const float* __restrict__ la, float* part,
+                                               int M, int K, int R, int m0) {
+    const int outs = ROWS * R, slices = lora_slices<THREADS>(K, outs), runs = K >> 2;
+    const int slice = static_cast<int>(threadIdx.x) / outs, out = static_cast<int>(threadIdx.x) % outs;
+    if (slice >= slices) return;
+    const float* xr = x + static_cast<size_t>(min(m0 + out / R, M - 1)) * K;
+    const float* lr = la + out % R;
+    part[threadIdx.x] = 4 * slices >= runs ? lora_rows_slice<4>(xr, lr, R, slice, slices, runs)
+                                           : lora_rows_slice<kLoraRuns>(xr, lr, R, slice, slices, runs);
+}
+template <int ROWS, int THREADS>
+__device__ __forceinline__ float lora_rows_sum(const float* part, int K, int R) {
+    const int outs = ROWS * R, slices = lora_slices<THREADS>(K, outs);
+    double s = 0.0;
+    if (static_cast<int>(threadIdx.x) < outs) {
+        for (int i0 = 0; i0 < slices; i0 += 4) {
+            float p[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[i] = part[min(i0 + i, slices - 1) * outs + static_cast<int>(threadIdx.x)];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (i0 + i < slices) s += static_cast<double>(p[i]);
+        }
+    }
+    return static_cast<float>(s);
+}
+
 // LoRA pre-pass on the MFMA: tpart[z][m][r] = sum over the kLoraGroupsPerBlock groups
 // of split z of x[m][k] * la[k][r] (la is K x R row-major). One workgroup of 4
 // wavefronts per 16 x 16 tile of (rows, ranks) and split; each wavefront takes

@@ -191,13 +191,13 @@ __device__ float ieee_row_value(const float* x, const uint32_t* wq, const float*
 // NI: output register pairs per lane in use (rows 2 i + h, i < NI): 1 for M <= 2, 2 for M <= 4,
 // else 4. W: wavefronts per workgroup, splitting K. Every variant keeps four wavefronts per SIMD
 // resident (at most 128 VGPRs and 40 KiB of LDS per wavefront), which hides the recoding's
-// dependent chains. Taken for short K and for some grids of one tile per CU (plan_digit_tiles).
-template <int NI, int W>
+// dependent chains. OWN_T: a LoRA call whose T the workgroup computes itself. Taken for short K and for some grids of one tile per CU (plan_digit_tiles).
+template <int NI, int W, bool OWN_T>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void q4_gemm_small_kernel(const float* x, const uint32_t* wq, const float* ws,
                                                                float* __restrict__ y, int M, int N, int K, int RB,
-                                                               int tiles_n, const float* __restrict__ tpart,
-                                                               int t_splits, const float* __restrict__ lb, int R,
-                                                               float lscale) {
+                                                               int tiles_n, const float* __restrict__ la,
+                                                               const float* __restrict__ tpart, int t_splits,
+                                                               const float* __restrict__ lb, int R, float lscale) {
     __shared__ __align__(16) unsigned char stages[kStages * W * kStageBytes];
     __shared__ __align__(16) int exps[W * kChunk * kDigitRows];
     __shared__ int rowmask;
@@ -219,6 +219,13 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
     const int n0 = (lin / RB) * kDigitCols;
     const int m0 = rb * kDigitRows;
     if (threadIdx.x == 0) rowmask = 0;
+    float t_own = 0.0f;     // element threadIdx.x of the workgroup's T
+    if constexpr (OWN_T) {  // slices in the stages, not yet in use
+        float* part = reinterpret_cast<float*>(stages);
+        lora_rows_load<kDigitRows, 64 * W>(x, la, part, M, K, R, m0);
+        __syncthreads();
+        t_own = lora_rows_sum<kDigitRows, 64 * W>(part, K, R);
+    }
     __syncthreads();
 
     // The workgroup's K range in chunks of kChunk groups, dealt to its wavefronts in turn (wave w
@@ -428,6 +435,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
     float* lora_b_s = lora_t_s + kDigitRows * kMaxLoraRank;  // [R][32 columns]
 #pragma unroll
     for (int i = 0; i < NI; ++i) red[(w * NI + i) * 64 + lane] = acc[i];
+    if (OWN_T && static_cast<int>(threadIdx.x) < kDigitRows * R) lora_t_s[threadIdx.x] = t_own;
     if (lb != nullptr) {
         // T (8 rows) and lb (32 columns): every load of a pass issued before the first store.
         constexpr int kNV = 2;
@@ -438,11 +446,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) voi
                 const int e = e0 + 64 * W * v;
                 bv[v] = lb[static_cast<size_t>(min(e >> 5, R - 1)) * N + min(n0 + (e & 31), N - 1)];  // in bounds
             }
-            lora_t_values<kNV>(tpart, t_splits, M, R, 0, R, m0, e0, 64 * W, kDigitRows * R, tv);
+            if constexpr (!OWN_T) lora_t_values<kNV>(tpart, t_splits, M, R, 0, R, m0, e0, 64 * W, kDigitRows * R, tv);
 #pragma unroll
             for (int v = 0; v < kNV; ++v) {
                 const int e = e0 + 64 * W * v;
-                if (e < kDigitRows * R) lora_t_s[e] = tv[v];
+                if (!OWN_T && e < kDigitRows * R) lora_t_s[e] = tv[v];
                 if (e < R * kDigitCols) lora_b_s[e] = bv[v];
             }
         }
@@ -752,6 +760,17 @@ __global__ __launch_bounds__(64 * kTileWaves) void q4_gemm_tiles_kernel(const fl
 
 }  // namespace
 
+// Whether q4_gemm_small_kernel computes T itself (at the workgroup size it will have). A chain of 128 x 64
+// -> 192 and -> 64 with rank 8 and -> 320 without: 24.5 us per graph replay with the two T launches,
+// 21.3 without.
+bool digits_lora_in_kernel(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, uint32_t rank) {
+    const size_t total = static_cast<size_t>((m + kDigitRows - 1) / kDigitRows) * ((n + kDigitCols - 1) / kDigitCols);
+    const size_t cus = static_cast<size_t>(dev.cu_count);
+    return total <= cus       ? lora_in_kernel<kDigitRows, 1024>(k, rank)
+           : total <= 2 * cus ? lora_in_kernel<kDigitRows, 512>(k, rank)
+                              : lora_in_kernel<kDigitRows, 256>(k, rank);
+}
+
 // Estimate fitted to the measured calls of 3 to 512 rows: per round of workgroups on the CUs and unit of
 // (CT + 2) tiles (recoding costs as much as about two tiles), 0.61 us for each chunk of a wavefront plus
 // 0.3; below one chunk per wavefront the fixed part of a workgroup, 0.6. CT is the one with the
@@ -799,7 +818,11 @@ hipError_t launch_q4gemm_small(const DeviceInfo& dev, const float* x, const uint
     const int RB = (M + kDigitRows - 1) / kDigitRows;
     const int R = static_cast<int>(rank);
     float* tpart = nullptr;
-    if (rank) {
+    const int tiles_n = (N + kDigitCols - 1) / kDigitCols;
+    // 16 wavefronts per CU in total, whether one, two or four workgroups of the small kernel share it
+    const size_t total = static_cast<size_t>(RB) * tiles_n;
+    const int W = total <= static_cast<size_t>(dev.cu_count) ? 16 : total <= 2 * static_cast<size_t>(dev.cu_count) ? 8 : 4;
+    if (t_splits > 0) {
         tpart = static_cast<float*>(workspace);
         const int tiles_m_t = (M + 15) / 16, tiles_r = (R + 15) / 16;
         hipLaunchKernelGGL(small_lora_prep_kernel, dim3(static_cast<unsigned>(tiles_m_t * tiles_r * t_splits)),
@@ -807,21 +830,23 @@ hipError_t launch_q4gemm_small(const DeviceInfo& dev, const float* x, const uint
         const hipError_t pe = hipGetLastError();
         if (pe != hipSuccess) return pe;
     }
-    const int tiles_n = (N + kDigitCols - 1) / kDigitCols;
     const float* lbp = rank ? lb : nullptr;
     const uint32_t* wq = reinterpret_cast<const uint32_t*>(w_packed);
     auto go = [&](auto ct, auto ni) {
         constexpr int CT = decltype(ct)::value, NI = decltype(ni)::value;
         if constexpr (CT == 0) {
-            // 16 wavefronts per CU in total, whether one, two or four workgroups share it
-            const size_t total = static_cast<size_t>(RB) * tiles_n;
             auto small = [&](auto wv) {
-                constexpr int W = decltype(wv)::value;
-                hipLaunchKernelGGL((q4_gemm_small_kernel<NI, W>), dim3(static_cast<unsigned>(total)), dim3(64 * W), 0, stream, x,
-                                   wq, w_scales, y, M, N, K, RB, tiles_n, tpart, t_splits, lbp, R, lora_scale);
+                constexpr int WV = decltype(wv)::value;
+                auto launch = [&](auto own) {
+                    hipLaunchKernelGGL((q4_gemm_small_kernel<NI, WV, decltype(own)::value>), dim3(static_cast<unsigned>(total)),
+                                       dim3(64 * WV), 0, stream, x, wq, w_scales, y, M, N, K, RB, tiles_n, la, tpart,
+                                       t_splits, lbp, R, lora_scale);
+                };
+                if (rank && t_splits == 0) launch(std::true_type{});
+                else launch(std::false_type{});
             };
-            if (total <= static_cast<size_t>(dev.cu_count)) small(std::integral_constant<int, 16>{});
-            else if (total <= 2 * static_cast<size_t>(dev.cu_count)) small(std::integral_constant<int, 8>{});
+            if (W == 16) small(std::integral_constant<int, 16>{});
+            else if (W == 8) small(std::integral_constant<int, 8>{});
             else small(std::integral_constant<int, 4>{});
         } else {
             const int blocks_n = (tiles_n + CT - 1) / CT;

@@ -54,7 +54,11 @@ def test_shapes(session, oracle, gpu, m, n, k):
     assert rep["status"] == "pass", rep
 
 
-@pytest.mark.parametrize("m,n,k,rank", [(40, 300, 1056, 5), (9, 9000, 544, 64), (128, 192, 64, 24), (100, 1030, 1024, 16)])
+@pytest.mark.parametrize("m,n,k,rank", [(40, 300, 1056, 5), (9, 9000, 544, 64), (128, 192, 64, 24), (100, 1030, 1024, 16),
+                                        # T in the kernel: 16, 8 and 4 wavefronts, uneven slices, a slice past
+                                        # the last run, one and 64 ranks, and the first K past it
+                                        (3, 40, 32, 1), (61, 70, 224, 11), (128, 64, 64, 64), (70, 1500, 96, 3),
+                                        (130, 3000, 64, 5), (17, 50, 416, 8), (17, 50, 544, 8)])
 def test_lora(session, oracle, gpu, m, n, k, rank):
     import torch
 
