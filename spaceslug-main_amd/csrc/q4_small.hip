@@ -780,6 +780,9 @@ DigitTiles plan_digit_tiles(const DeviceInfo& dev, uint32_t m, uint32_t n, uint3
     if (k > (1u << 22)) return {0, FLT_MAX};  // beyond 32-bit offsets of 256 columns
     const size_t rb = (m + kDigitRows - 1) / kDigitRows, tiles_n = (n + kDigitCols - 1) / kDigitCols;
     const size_t cus = static_cast<size_t>(dev.cu_count);
+    // q4_gemm_small_kernel keeps a short K, whose few chunks its smaller workgroups spread over more
+    // CUs (32 x 192 -> 10000 5.2 against 6.2 us; at K = 512 7.5 against 6.6).
+    if (k < 512) return {0, 3.2f + static_cast<float>(rb * tiles_n) * (1.0e-3f + 3.2e-6f * static_cast<float>(k))};
     size_t best = 0;
     int tiles = 0;
     for (int ct : {1, 2, 3, 4, 5, 6, 8}) {
@@ -789,12 +792,10 @@ DigitTiles plan_digit_tiles(const DeviceInfo& dev, uint32_t m, uint32_t n, uint3
             best = units;
             tiles = ct;
         }
+        if (rounds <= 1) break;  // more tiles would only lengthen it
     }
     const float chunks = static_cast<float>((k / kGroup + kTileGroups - 1) / kTileGroups) / kTileWaves;
     const float us = 2.8f + static_cast<float>(best) * std::max(0.6f, 0.3f + 0.61f * (chunks < 1.0f ? chunks : std::ceil(chunks)));
-    // q4_gemm_small_kernel keeps a short K, whose few chunks its smaller workgroups spread over more
-    // CUs (32 x 192 -> 10000 5.2 against 6.2 us; at K = 512 7.5 against 6.6).
-    if (k < 512) return {0, 3.2f + static_cast<float>(rb * tiles_n) * (1.0e-3f + 3.2e-6f * static_cast<float>(k))};
     // With one tile per workgroup it also keeps
     //   - K below 3072, unless the chunks fill whole rounds of the wavefronts: its shorter chunks divide
     //     more evenly (16 -> 4000 columns: K = 1024 4.6 against 4.8 us, 2688 7.7 against 7.8; but 2048 6.8
