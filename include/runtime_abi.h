@@ -188,8 +188,9 @@ void spaceslug_q4_weight_destroy(spaceslug_q4_weight* weight);
 int spaceslug_q4gemm_run(const spaceslug_q4_weight* weight, const float* x, float* y, uint32_t m);
 
 /* Retained projection chain: a fixed sequence of device-pointer projections recorded
- * once into one HIP graph and replayed with one launch, with no host round trip and
- * no per-call planning between the steps. Replaces the reference's retained
+ * once into one HIP graph and replayed with one call, with no host round trip and
+ * no per-call planning between the steps (a chain of at most 6 kernels enqueues them
+ * itself where the stream is not capturing: a graph launch costs more). Replaces the reference's retained
  * command buffers (vulkan-runtime/src/exec/engine.h:85-101, recordImmutable /
  * submitImmutable: "retain fully recorded command buffers and resubmit without
  * re-recording") and the persistent tiny forward's handle pattern

@@ -893,7 +893,6 @@ constexpr int kWideTile = 128;
 
 size_t align_up(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
-
 }  // namespace
 
 size_t split_x_bf16_bytes(uint32_t m, uint32_t k) {

@@ -55,6 +55,16 @@ struct DeviceInfo {
 // Decides the kernel and K-split for (m, n, k, rank). rank == 0 means no LoRA.
 Q4Plan plan_q4gemm(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, uint32_t rank);
 
+// Kernel launches of launch_q4gemm for a plan.
+constexpr int plan_launches(const Q4Plan& p) {
+    switch (p.kind) {
+        case Q4Plan::kGemv: return 1;
+        case Q4Plan::kDigits: return p.t_splits > 0 ? 2 : 1;
+        case Q4Plan::kMid: return 2;
+        default: return p.splits > 1 ? 3 : 2;
+    }
+}
+
 // Decode GEMV for the shapes gemv_takes accepts (no device memory beyond its arguments).
 hipError_t launch_gemv(const DeviceInfo& dev, const float* x, const uint8_t* w_packed,
                        const float* w_scales, float* y, uint32_t m, uint32_t n, uint32_t k,

@@ -347,12 +347,17 @@ struct spaceslug_q4_weight {
     float* d_scales;
 };
 
-// A retained chain: the instantiated graph of its steps' launches and the device
-// workspace those launches were recorded against (owned by the chain, so a replay
-// shares no memory with any other call).
+// A retained chain: its validated steps with their plans, the instantiated graph of
+// their launches and the device workspace those launches were recorded against (owned
+// by the chain, so a replay shares no memory with any other call).
 struct spaceslug_q4_chain {
     int device = -1;
-    uint32_t steps = 0;
+    std::vector<spaceslug_q4_step> steps;
+    std::vector<spaceslug::Q4Plan> plans;
+    spaceslug::DeviceInfo info{};
+    bool direct = false;  // few launches: a replay enqueues them itself
+    std::mutex enqueue;   // one replay at a time: neither single launches nor a graph's are kept from
+                          // interleaving with another thread's by the stream alone
     void* workspace = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -375,6 +380,25 @@ const char* device_call_problem(const float* d_x, const uint8_t* d_w_packed, con
         if (!aligned(d_lora_a, 4) || !aligned(d_lora_b, 4)) return "misaligned device pointer";
     }
     return nullptr;
+}
+
+// Replaying a graph costs the host ~18 us and the GPU ~4 us beyond its kernels however few they are,
+// a kernel launch ~3 us of host time: up to this many launches a replay enqueues them one by one.
+// Graph against direct, us per replay of a chain of 1 x 4096 -> 4096 back to back, and of one alone until
+// it is done: 1 step 22.5 -> 3.9 (33 -> 15), 2 steps 15.7 -> 8.1 (34 -> 19), 4 steps 22.0 -> 15.7 (36 -> 27),
+// 8 steps 37.3 -> 31.8 (49 -> 61), 16 steps 68.7 -> 63.1 (80 -> 80): past the line the replay alone loses.
+constexpr int kDirectLaunches = 6;
+
+// Enqueues a chain's steps on `st`, in order (a replay, or the recording of its graph).
+void chain_enqueue(const spaceslug_q4_chain& c, hipStream_t st) {
+    for (size_t i = 0; i < c.steps.size(); ++i) {
+        const spaceslug_q4_step& s = c.steps[i];
+        const bool lora = s.d_lora_a != nullptr;
+        check(spaceslug::launch_q4gemm(c.plans[i], c.info, s.d_x, s.d_w_packed, s.d_w_scales, s.d_y, s.m, s.n, s.k,
+                                       s.d_lora_a, s.d_lora_b, lora ? s.rank : 0, lora ? s.lora_scale : 0.0f,
+                                       c.workspace, st),
+              "q4gemm launch (chain)");
+    }
 }
 
 // Releases whatever a partly built chain holds (the device is current).
@@ -745,27 +769,22 @@ spaceslug_q4_chain* spaceslug_q4_chain_create(const spaceslug_q4_step* steps, ui
         DeviceState& dev = current_device();
         c = new spaceslug_q4_chain;
         check(hipGetDevice(&c->device), "hipGetDevice");
-        c->steps = count;
-        std::vector<spaceslug::Q4Plan> plans;
+        c->steps.assign(steps, steps + count);
+        c->info = dev.info;
         size_t ws = 0;
-        for (uint32_t i = 0; i < count; ++i) {
-            const spaceslug_q4_step& s = steps[i];
-            plans.push_back(spaceslug::plan_q4gemm(dev.info, s.m, s.n, s.k, s.d_lora_a ? s.rank : 0));
-            ws = std::max(ws, plans.back().workspace_bytes);
+        int launches = 0;
+        for (const spaceslug_q4_step& s : c->steps) {
+            c->plans.push_back(spaceslug::plan_q4gemm(dev.info, s.m, s.n, s.k, s.d_lora_a ? s.rank : 0));
+            ws = std::max(ws, c->plans.back().workspace_bytes);
+            launches += spaceslug::plan_launches(c->plans.back());
         }
+        c->direct = launches <= kDirectLaunches;
         // The steps run one after another inside the graph, so one workspace serves all of them.
         if (ws) check(hipMalloc(&c->workspace, ws), "hipMalloc (chain workspace)");
         check(hipStreamCreateWithFlags(&capture, hipStreamNonBlocking), "hipStreamCreateWithFlags");
         check(hipStreamBeginCapture(capture, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         capturing = true;
-        for (uint32_t i = 0; i < count; ++i) {
-            const spaceslug_q4_step& s = steps[i];
-            const bool lora = s.d_lora_a != nullptr;
-            check(spaceslug::launch_q4gemm(plans[i], dev.info, s.d_x, s.d_w_packed, s.d_w_scales, s.d_y, s.m, s.n, s.k,
-                                           s.d_lora_a, s.d_lora_b, lora ? s.rank : 0, lora ? s.lora_scale : 0.0f,
-                                           c->workspace, capture),
-                  "q4gemm launch (capture)");
-        }
+        chain_enqueue(*c, capture);
         capturing = false;
         check(hipStreamEndCapture(capture, &c->graph), "hipStreamEndCapture");
         check(hipGraphInstantiate(&c->exec, c->graph, nullptr, nullptr, 0), "hipGraphInstantiate");
@@ -796,7 +815,19 @@ int spaceslug_q4_chain_run(spaceslug_q4_chain* chain, void* stream) {
         check(hipGetDevice(&cur), "hipGetDevice");
         if (cur != chain->device)
             return fail(SPACESLUG_ERR_INVALID, "spaceslug_q4_chain_run: chain lives on another device");
-        check(hipGraphLaunch(chain->exec, static_cast<hipStream_t>(stream)), "hipGraphLaunch");
+        const hipStream_t st = static_cast<hipStream_t>(stream);
+        std::lock_guard<std::mutex> lock(chain->enqueue);
+        if (chain->direct) {
+            // Single launches would be recorded by a stream that is capturing, which the graph's launch is not:
+            // the graph there, and wherever the query has no answer.
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
+                chain_enqueue(*chain, st);
+                return ok();
+            }
+            (void)hipGetLastError();
+        }
+        check(hipGraphLaunch(chain->exec, st), "hipGraphLaunch");
         return ok();
     } catch (const HipError& e) {
         return from_hip(e);

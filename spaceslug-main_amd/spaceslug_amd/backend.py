@@ -149,8 +149,8 @@ class Q4Step(ctypes.Structure):
 
 
 class Q4Chain:
-    """A retained chain of device-pointer projections replayed as one HIP graph
-    (spaceslug_q4_chain_create / _run / _destroy). The buffers named by the steps must
+    """A retained chain of device-pointer projections replayed with one call, as one HIP graph or, for a
+    few kernels, launch by launch (spaceslug_q4_chain_create / _run / _destroy). The buffers named by the steps must
     outlive the chain; refill their contents between runs, never move them."""
 
     def __init__(self, session: "BackendSession", handle: int, steps: int) -> None:

@@ -100,6 +100,58 @@ def test_chain_replays_equal_eager_calls(session, oracle, gpu):
         chain.close()
 
 
+@pytest.mark.parametrize("steps", [1, 3, 6, 7, 9])
+def test_chain_of_one_launch_per_step(session, oracle, gpu, steps):
+    """Either side of the line between direct launches and the graph: a chain whose last step writes the
+    first one's input, so that each replay depends on the one before, replayed by two threads at once on one
+    stream (in either order the same sequence), against eager calls bit for bit."""
+    import threading
+
+    import torch
+
+    note(f"chain of {steps} launches")
+    h, dev = 512, torch.device("cuda:0")
+    rng = np.random.default_rng(steps)
+    ws = []
+    for _ in range(steps):
+        p, s = oracle.q4_quantize(rand(rng, h, h, scale=0.045))
+        ws.append((torch.from_numpy(p).to(dev), torch.from_numpy(s).to(dev)))
+    start = torch.from_numpy(rand(rng, 3, h)).to(dev)
+    bufs = [torch.empty_like(start) for _ in range(max(2, steps))]  # step i reads bufs[i], writes bufs[i + 1]
+    spare = torch.empty_like(start)
+
+    def dest(i):
+        return (spare if steps == 1 else bufs[0]) if i == steps - 1 else bufs[i + 1]
+
+    spec = [{"d_x": bufs[i].data_ptr(), "d_w_packed": ws[i][0].data_ptr(), "d_w_scales": ws[i][1].data_ptr(),
+             "d_y": dest(i).data_ptr(), "m": 3, "n": h, "k": h} for i in range(steps)]
+    st = torch.cuda.Stream()
+
+    def eager(runs):
+        bufs[0].copy_(start)
+        torch.cuda.synchronize()
+        for _ in range(runs):
+            for s in spec:
+                session.q4gemm_device(s["d_x"], s["d_w_packed"], s["d_w_scales"], s["d_y"], 3, h, h, st.cuda_stream)
+        torch.cuda.synchronize()
+        return dest(steps - 1).clone()
+
+    chain = session.create_q4_chain(spec)
+    try:
+        want = eager(16)
+        bufs[0].copy_(start)
+        torch.cuda.synchronize()
+        threads = [threading.Thread(target=lambda: [chain.run(st.cuda_stream) for _ in range(8)]) for _ in range(2)]
+        for th in threads:
+            th.start()
+        for th in threads:
+            th.join()
+        torch.cuda.synchronize()
+        assert torch.equal(dest(steps - 1), want) and torch.isfinite(want).all()
+    finally:
+        chain.close()
+
+
 def test_chain_rejects_run_on_closed_handle(session, gpu):
     import torch
 
