@@ -375,6 +375,67 @@ __global__ __launch_bounds__(256) void cq4_transform_orthogonal_kernel(Cq4View w
     store_code(out, lo, w.K, m, i, acc);
 }
 
+// The same for K % 16 == 0 and 8-byte aligned arrays, on the fp32 matrix cores: the kernel above runs one
+// chain of K dependent loads and FMAs per output, 157 us at K = 1024 however few the rows. What bounds this
+// one is latency up to about a hundred rows (every load of K <= 1024 is in flight at once), the fp32 MFMA
+// rate above. Whole calls, before and after: 1 x 1024 -> 4096 190 -> 13.3 us, 8 x 1024 -> 1024 in panels 242 -> 14.8,
+// 200 x 768 -> 1024 173 -> 23.7, 1024^3 571 -> 54.6, 2 x 4096 -> 4096 1786 -> 36.6. A workgroup of 16 wavefronts owns 16 rows x 64 columns; wavefront v takes every 16th step
+// of 16 values of k from v on, and their 16 sums are added in double, in order (chains of K / 16 instead
+// of K products in fp32). MFMA j of a step takes k = 4 * quarter + j on both operands, so a lane loads
+// its four x and four scales as one run each, and column tile t is columns 4 c + t, so that it loads four
+// columns of a row of R at once; columns past K repeat the last four and are not stored.
+constexpr uint32_t kOrthRows = 16, kOrthCols = 64, kOrthWaves = 16, kOrthDepth = 4;
+__global__ __launch_bounds__(64 * kOrthWaves) void cq4_transform_orthogonal_mfma_kernel(Cq4View w,
+                                                                                       const uint16_t* __restrict__ a,
+                                                                                       float* __restrict__ out,
+                                                                                       Cq4LimbOut lo, uint32_t M,
+                                                                                       uint32_t tiles_m) {
+    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+    __shared__ float red[kOrthWaves][kOrthRows][kOrthCols];
+    const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x % 64, c = lane % 16, q = lane / 16;
+    const uint32_t m0 = blockIdx.x % tiles_m * kOrthRows, n0 = blockIdx.x / tiles_m * kOrthCols;
+    const uint16_t* ar = a + static_cast<size_t>(min(m0 + c, M - 1)) * w.K + 4 * q;
+    const uint16_t* sr = w.input_scale_recip ? w.input_scale_recip : w.input_scale;
+    const uint16_t* rr = w.rotation + static_cast<size_t>(4 * q) * w.K + min(n0 + 4 * c, w.K - 4);
+    const uint32_t steps = w.K / 16;
+    f32x4 acc[4] = {};
+    for (uint32_t s0 = wave; s0 < steps; s0 += kOrthWaves * kOrthDepth) {
+        u16x4 x[kOrthDepth], sc[kOrthDepth], r[kOrthDepth][4];
+#pragma unroll
+        for (uint32_t d = 0; d < kOrthDepth; ++d) {
+            const uint32_t k = 16 * min(s0 + d * kOrthWaves, steps - 1);  // past the last: in bounds, not used
+            x[d] = *reinterpret_cast<const u16x4*>(ar + k);
+            if (sr) sc[d] = *reinterpret_cast<const u16x4*>(sr + 4 * q + k);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                r[d][j] = *reinterpret_cast<const u16x4*>(rr + static_cast<size_t>(k + j) * w.K);
+        }
+#pragma unroll
+        for (uint32_t d = 0; d < kOrthDepth; ++d) {
+            if (s0 + d * kOrthWaves >= steps) break;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float xv = half_bits_to_float(x[d][j]);
+                if (w.input_scale_recip) xv *= half_bits_to_float(sc[d][j]);
+                else if (sr) xv *= 1.0f / half_bits_to_float(sc[d][j]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv, half_bits_to_float(r[d][j][t]), acc[t], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<f32x4*>(&red[wave][4 * q + i][4 * c]) = f32x4{acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
+    __syncthreads();
+    const uint32_t row = wave, col = lane;
+    if (m0 + row >= M || n0 + col >= w.K) return;
+    double sum = 0.0;
+#pragma unroll
+    for (uint32_t v = 0; v < kOrthWaves; ++v) sum += static_cast<double>(red[v][row][col]);
+    store_code(out, lo, w.K, m0 + row, n0 + col, static_cast<float>(sum));
+}
+
 // Index k of a row's LSB-first group (cactus_x86.cpp:24-43), any bits in 1..4.
 __device__ __forceinline__ uint32_t index_lsb(const uint8_t* p, uint32_t k, uint32_t bits) {
     const uint32_t bit = k * bits;
@@ -1525,7 +1586,13 @@ hipError_t launch_cq4_matmul(const Cq4View& w, const uint16_t* a, uint32_t m, ui
     float* ap = limbs ? nullptr : static_cast<float*>(workspace);
     const Cq4LimbOut lo{limbs ? static_cast<uint16_t*>(workspace) : nullptr, plan.layout, inter};
     const uint32_t gs = orth ? w.K : w.group_size, ng = orth ? 1 : w.num_groups;
-    if (orth) {
+    if (orth && w.K % 16 == 0 && aligned(a, 8) && aligned(w.rotation, 8) && aligned(w.input_scale_recip, 8) &&
+        aligned(w.input_scale, 8)) {
+        const uint32_t tiles_m = (m + kOrthRows - 1) / kOrthRows;
+        const dim3 grid(tiles_m * ((w.K + kOrthCols - 1) / kOrthCols));
+        hipLaunchKernelGGL(cq4_transform_orthogonal_mfma_kernel, grid, dim3(64 * kOrthWaves), 0, stream, w, a, ap, lo, m,
+                           tiles_m);
+    } else if (orth) {
         hipLaunchKernelGGL(cq4_transform_orthogonal_kernel, dim3((w.K + 255) / 256, m), dim3(256), 0, stream, w, a,
                            ap, lo);
     } else if (limbs && aligned(a, 16) && aligned(w.input_scale_recip, 16) && aligned(w.input_scale, 16) &&

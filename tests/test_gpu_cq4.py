@@ -320,3 +320,17 @@ def test_batch_nonfinite_follows_ieee(session, gpu, interleaved, K, gs, m):
         ok = np.isfinite(ref)
         assert ok.any() == (code is None)
         assert np.all(np.abs(got[ok] - ref[ok]) <= 2.0 ** -11 * np.abs(ref[ok]) + 1e-5 * np.maximum(1, np.abs(ref[ok])))
+
+
+# The rotation on the matrix cores (K % 16 == 0): fewer steps than wavefronts, one and several passes, the
+# last pass partly empty, column and row tiles that are ragged or exactly full, every limb layout, both scale
+# forms; K = 100 on the other kernel.
+@pytest.mark.parametrize("K,m,kw", [(16, 1, {}), (16, 17, dict(scale="none")), (48, 3, {}), (64, 16, dict(interleaved=True)),
+                                    (100, 5, {}), (240, 33, dict(scale="scale")), (256, 4, dict(interleaved=True)),
+                                    (272, 2, dict(bits=3)), (1008, 6, {}), (1024, 65, dict(interleaved=True)),
+                                    (1040, 1, dict(scale="scale")), (2064, 31, {})])
+def test_orthogonal_rotation(session, gpu, K, m, kw):
+    rng = np.random.default_rng(77 + K)
+    W = cq4.random_matrix(rng, **{**dict(bits=4, K=K, N=20, group_size=K, orthogonal=True), **kw})
+    A = cq4.f16(rng.uniform(-1, 1, (m, K)))
+    check(session, W, A, m, f"orthogonal K={K} m={m} {kw}")
