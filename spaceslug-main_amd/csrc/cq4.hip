@@ -617,73 +617,138 @@ __global__ __launch_bounds__(256) void cq4_gemv_kernel(Cq4View w, const float* _
 
 // Rows x K values the fused GEMV transforms in LDS (two arrays of that many floats: 32 KiB).
 constexpr uint32_t kCq4FusedMaxValues = 4096;
+// Index words of a column per lane: K <= kCq4FusedMaxValues.
+constexpr uint32_t kCq4FusedWords = kCq4FusedMaxValues / 512;
+
+template <int MASK>
+__device__ __forceinline__ void butterfly_lanes(float (&v)[8], uint32_t lane) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float o = lane_xor<MASK>(v[e]);
+        v[e] = (lane & MASK) ? o - v[e] : v[e] + o;
+    }
+}
 
 // The GEMV above with the Hadamard transform in the same launch (M <= 4, power-of-two group
-// size <= 256, M * K <= kCq4FusedMaxValues): every workgroup transforms all M rows into LDS with
+// size 8 to 256, M * K <= kCq4FusedMaxValues): every workgroup transforms all M rows into LDS with
 // the operations of cq4_transform_hadamard_kernel, in the same order (scale and left sign, the
 // butterflies of strides 1 .. gs / 2, then the permuted, normalized, right-signed values), so
-// its four wavefronts read exactly the values the two-launch form reads from memory, and run
-// its columns. Each lane's first index word and norm are loaded before the transform, so their
-// latency overlaps it; the call needs no workspace and one launch instead of two. Dynamic LDS:
-// 2 * M * K floats.
-template <int ROWS, bool INTER>
-__global__ __launch_bounds__(256) void cq4_gemv_fused_kernel(Cq4View w, const uint16_t* __restrict__ a,
-                                                            uint16_t* __restrict__ c, uint32_t M, uint32_t gs,
-                                                            uint32_t ng) {
+// its W wavefronts read exactly the values the two-launch form reads from memory, and run
+// its columns. The call needs no workspace and one launch instead of two. Dynamic LDS: 2 * M * K floats.
+// What bounds it is the transform that every workgroup repeats, and latency. So a wavefront keeps 512
+// values of the transform in registers, eight per lane (a group never leaves it: strides of 8 and more pair
+// lanes), instead of a barrier per stage, all of a lane's index words and norms of its first column are
+// loaded before the transform (the next column's as each is used), and W is 16 where the columns fill the chip:
+// 1 x 4096 -> 4096 19.6 -> 8.2 us, 1 x 4096 -> 8192 37.9 -> 12.2, 4 x 1024 -> 4096 in panels 22.3 -> 9.0, 1 x 512 -> 512 4.5.
+template <int ROWS, bool INTER, int W>
+__global__ __launch_bounds__(64 * W) void cq4_gemv_fused_kernel(Cq4View w, const uint16_t* __restrict__ a,
+                                                               uint16_t* __restrict__ c, uint32_t M, uint32_t gs,
+                                                               uint32_t ng, bool vec) {
     extern __shared__ f32x4_t fused_lds[];
     __shared__ float lut[16];
-    const uint32_t tid = threadIdx.x, lane = tid & 63;
-    const uint32_t n = blockIdx.x * 4 + (tid >> 6);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t K = w.K, words = K >> 3, wpg = gs >> 3, total = M * K;
-    float* xv = reinterpret_cast<float*>(fused_lds);  // scaled, signed, then transformed in place
+    float* xv = reinterpret_cast<float*>(fused_lds);  // transformed, for the permutation's gather
     float* xa = xv + total;                            // code-basis activations, row-major
     if (tid < 16) lut[tid] = half_bits_to_float(w.codebook[tid]);
-    const bool live = n < w.N;  // uniform per wavefront; every wavefront takes part in the transform
-    uint32_t word0 = 0;
-    uint16_t norm0 = 0;
-    if (live && lane < words) {
+    uint32_t n = blockIdx.x * W + wave;  // uniform per wavefront; every wavefront takes part in the transform
+    uint32_t word[kCq4FusedWords];
+    uint16_t norm[kCq4FusedWords];
+    auto load_word = [&](uint32_t i) {
         size_t ni;
-        word0 = cq4_gemv_word<INTER>(w, n, lane, wpg, ng, ni);
-        norm0 = w.norms[ni];
-    }
-    for (uint32_t e = tid; e < total; e += 256) {
-        const uint32_t k = e % K;
-        const float sign = w.left_signs ? static_cast<float>(w.left_signs[k % gs]) : 1.0f;
-        xv[e] = half_bits_to_float(a[e]) * input_recip(w, k) * sign;
+        word[i] = cq4_gemv_word<INTER>(w, n, min(lane + 64 * i, words - 1), wpg, ng, ni);
+        norm[i] = w.norms[ni];
+    };
+#pragma unroll
+    for (uint32_t i = 0; i < kCq4FusedWords; ++i)
+        if (n < w.N && 64 * i < words) load_word(i);
+    const uint16_t* sp = w.input_scale_recip ? w.input_scale_recip : w.input_scale;
+    const float inv = 1.0f / sqrtf(static_cast<float>(gs));
+    for (uint32_t e0 = wave * 512; e0 < total; e0 += W * 512) {
+        const uint32_t at = e0 + 8 * lane;  // past the end: lanes of no group, that load and store nothing
+        const bool live = at < total;
+        const uint32_t k = at - (at >= K ? K : 0) - (at >= 2 * K ? K : 0) - (at >= 3 * K ? K : 0);
+        const uint32_t j = k & (gs - 1);
+        float v[8] = {};
+        int8_t rs[8] = {};
+        if (live) {
+            uint16_t av[8], sv[8];
+            int8_t ls[8];
+            if (vec) {
+                *reinterpret_cast<u32x4*>(av) = *reinterpret_cast<const u32x4*>(a + at);
+                if (sp) *reinterpret_cast<u32x4*>(sv) = *reinterpret_cast<const u32x4*>(sp + k);
+                if (w.left_signs) *reinterpret_cast<uint2*>(ls) = *reinterpret_cast<const uint2*>(w.left_signs + j);
+                if (w.right_signs) *reinterpret_cast<uint2*>(rs) = *reinterpret_cast<const uint2*>(w.right_signs + j);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    av[e] = a[at + e];
+                    if (sp) sv[e] = sp[k + e];
+                    if (w.left_signs) ls[e] = w.left_signs[j + e];
+                    if (w.right_signs) rs[e] = w.right_signs[j + e];
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                // input_recip's value: the reciprocal as given, or 1 / scale, or 1
+                const float r = w.input_scale_recip ? half_bits_to_float(sv[e])
+                                                    : (w.input_scale ? 1.0f / half_bits_to_float(sv[e]) : 1.0f);
+                const float sign = w.left_signs ? static_cast<float>(ls[e]) : 1.0f;
+                v[e] = half_bits_to_float(av[e]) * r * sign;
+            }
+        }
+#pragma unroll
+        for (int h = 1; h < 8; h <<= 1)  // butterflies over strides 1, 2, 4, ... (cactus_x86.cpp:56-66)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if ((e & h) == 0) {
+                    const float x = v[e], y = v[e + h];
+                    v[e] = x + y;
+                    v[e + h] = x - y;
+                }
+        if (gs > 8) butterfly_lanes<1>(v, lane);
+        if (gs > 16) butterfly_lanes<2>(v, lane);
+        if (gs > 32) butterfly_lanes<4>(v, lane);
+        if (gs > 64) butterfly_lanes<8>(v, lane);
+        if (gs > 128) butterfly_lanes<16>(v, lane);
+        if (w.permutation == nullptr) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[e] = v[e] * inv * (w.right_signs ? static_cast<float>(rs[e]) : 1.0f);
+        }
+        if (live) {
+            f32x4_t* d = reinterpret_cast<f32x4_t*>((w.permutation ? xv : xa) + at);
+            d[0] = f32x4_t{v[0], v[1], v[2], v[3]};
+            d[1] = f32x4_t{v[4], v[5], v[6], v[7]};
+        }
     }
     __syncthreads();
-    for (uint32_t h = 1; h < gs; h <<= 1) {  // butterflies over strides 1, 2, 4, ... (cactus_x86.cpp:56-66)
-        // butterfly t pairs j and j + h inside one block of 2h values, so never across a group
-        for (uint32_t t = tid; t < total / 2; t += 256) {
-            const uint32_t j = (t / h) * 2 * h + (t % h);
-            const float x = xv[j], y = xv[j + h];
-            xv[j] = x + y;
-            xv[j + h] = x - y;
+    if (w.permutation) {
+        for (uint32_t e = tid; e < total; e += 64 * W) {
+            const uint32_t j = e & (gs - 1);  // K % gs == 0: the position inside the element's group
+            const uint32_t src = w.permutation[j] & (gs - 1);
+            const float sign = w.right_signs ? static_cast<float>(w.right_signs[src]) : 1.0f;
+            xa[e] = xv[e - j + src] * inv * sign;
         }
         __syncthreads();
     }
-    const float inv = 1.0f / sqrtf(static_cast<float>(gs));
-    for (uint32_t e = tid; e < total; e += 256) {
-        const uint32_t j = e % gs;  // K % gs == 0: the position inside the element's group
-        const uint32_t src = w.permutation ? (w.permutation[j] & (gs - 1)) : j;
-        const float sign = w.right_signs ? static_cast<float>(w.right_signs[src]) : 1.0f;
-        xa[e] = xv[e - j + src] * inv * sign;
-    }
-    __syncthreads();
-    if (!live) return;
     const float* arow[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) arow[r] = xa + min(static_cast<uint32_t>(r), M - 1) * K;
-    double acc[ROWS];
+    while (n < w.N) {
+        const uint32_t col = n;
+        n += gridDim.x * W;
+        double acc[ROWS];
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) acc[r] = 0.0;
-    if (lane < words) cq4_gemv_step<ROWS, INTER>(lut, word0, norm0, arow, lane, acc);
-    for (uint32_t wi = lane + 64; wi < words; wi += 64) {
-        size_t ni;
-        const uint32_t word = cq4_gemv_word<INTER>(w, n, wi, wpg, ng, ni);
-        cq4_gemv_step<ROWS, INTER>(lut, word, w.norms[ni], arow, wi, acc);
+        for (int r = 0; r < ROWS; ++r) acc[r] = 0.0;
+#pragma unroll
+        for (uint32_t i = 0; i < kCq4FusedWords; ++i) {
+            if (64 * i >= words) break;
+            if (lane + 64 * i < words) cq4_gemv_step<ROWS, INTER>(lut, word[i], norm[i], arow, lane + 64 * i, acc);
+            if (n < w.N) load_word(i);  // the next column's
+        }
+        cq4_gemv_store<ROWS>(acc, c, w.N, M, col, lane);
     }
-    cq4_gemv_store<ROWS>(acc, c, w.N, M, n, lane);
 }
 
 // MFMA form for 4-bit LSB-packed indices (the packing of cactus_x86.cpp:24-43 with
@@ -1567,16 +1632,31 @@ hipError_t launch_cq4_matmul(const Cq4View& w, const uint16_t* a, uint32_t m, ui
     const bool orth = (w.flags & kCq4FlagOrthogonal) != 0;
     const bool inter = (w.flags & kCq4FlagInterleaved4Row) != 0;
     if (cq4_gemv_fused(w, m)) {
-        const dim3 grid((w.N + 3) / 4);
+        // 16 columns a workgroup where that leaves about one workgroup per CU, or where the transform needs
+        // more than four wavefronts; 4, on more CUs, below (us per call, 16 against 4, one row: 1000 x 512
+        // 5.4, 4.6; 2500 x 1024 5.81, 5.85; 4096 x 2048 6.6, 7.8; 300 x 4096 8.8, 10.1). At most 16 wavefronts a
+        // CU: more would repeat the transform instead of looping over columns (6000 x 512: 6.2 against 10.1).
         const size_t lds = 2 * sizeof(float) * m * w.K;
         const uint32_t gs = w.group_size, ng = w.num_groups;
-        if (m == 1) {
-            if (inter) hipLaunchKernelGGL((cq4_gemv_fused_kernel<1, true>), grid, dim3(256), lds, stream, w, a, c, m, gs, ng);
-            else hipLaunchKernelGGL((cq4_gemv_fused_kernel<1, false>), grid, dim3(256), lds, stream, w, a, c, m, gs, ng);
-        } else {
-            if (inter) hipLaunchKernelGGL((cq4_gemv_fused_kernel<4, true>), grid, dim3(256), lds, stream, w, a, c, m, gs, ng);
-            else hipLaunchKernelGGL((cq4_gemv_fused_kernel<4, false>), grid, dim3(256), lds, stream, w, a, c, m, gs, ng);
-        }
+        const bool vec = aligned(a, 16) && aligned(w.input_scale_recip, 16) && aligned(w.input_scale, 16) &&
+                         aligned(w.left_signs, 8) && aligned(w.right_signs, 8);
+        auto go = [&](auto rows, auto panels, auto waves) {
+            constexpr int W = decltype(waves)::value;
+            const uint32_t blocks = (w.N + W - 1) / W;
+            hipLaunchKernelGGL((cq4_gemv_fused_kernel<decltype(rows)::value, decltype(panels)::value, W>),
+                               dim3(std::min(blocks, 4096u / W)), dim3(64 * W), lds, stream, w, a, c, m, gs,
+                               ng, vec);
+        };
+        auto by_rows = [&](auto panels, auto waves) {
+            if (m == 1) go(std::integral_constant<int, 1>{}, panels, waves);
+            else go(std::integral_constant<int, 4>{}, panels, waves);
+        };
+        auto by_waves = [&](auto panels) {
+            if (w.N > 2560 || m * w.K > 3072) by_rows(panels, std::integral_constant<int, 16>{});
+            else by_rows(panels, std::integral_constant<int, 4>{});
+        };
+        if (inter) by_waves(std::true_type{});
+        else by_waves(std::false_type{});
         return hipGetLastError();
     }
     // The transform writes the code-basis activations as fp32 rows, or, for the limb GEMMs, directly as

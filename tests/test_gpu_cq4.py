@@ -334,3 +334,33 @@ def test_orthogonal_rotation(session, gpu, K, m, kw):
     W = cq4.random_matrix(rng, **{**dict(bits=4, K=K, N=20, group_size=K, orthogonal=True), **kw})
     A = cq4.f16(rng.uniform(-1, 1, (m, K)))
     check(session, W, A, m, f"orthogonal K={K} m={m} {kw}")
+
+
+# Decode calls with the transform in the launch: both workgroup sizes (the line at 2560 columns or 3072
+# values), every group size, fewer values than one wavefront's 512, rows that end inside them, columns past
+# one per wavefront of the grid, panels, permutations, signs; arrays as they are and shifted by one element.
+@pytest.mark.parametrize("m,N,K,gs,kw", [(1, 3, 8, 8, dict(signs=True)), (3, 40, 16, 16, dict(signs=True, perm=True)),
+                                         (4, 24, 1024, 32, dict(signs=True, interleaved=True)), (2, 2561, 96, 8, dict(scale="scale")),
+                                         (1, 2560, 64, 64, dict(signs=True)), (3, 60, 1024, 256, dict(signs=True, perm=True)),
+                                         (1, 4101, 520, 8, dict(signs=True)), (2, 8200, 256, 128, dict(signs=True, interleaved=True)),
+                                         (3, 52, 1152, 128, dict(signs=True, scale="scale")), (1, 30, 4096, 16, dict(perm=True, scale="none")),
+                                         (4, 9000, 128, 64, dict(perm=True, signs=True))])
+def test_decode_transform_in_the_launch(session, gpu, m, N, K, gs, kw):
+    import torch
+
+    note(f"cq4 decode {m}x{K}->{N} gs={gs} {kw}")
+    rng = np.random.default_rng(31 + N + K)
+    W = cq4.random_matrix(rng, bits=4, K=K, N=N, group_size=gs, **kw)
+    A = cq4.f16(rng.uniform(-1, 1, (m, K)))
+    got = check(session, W, A, m, f"decode {m}x{K}->{N}")
+    keep = {}
+    s = device_struct(W, keep)
+    a_t = torch.from_numpy(A.view(np.int16).copy()).to("cuda:0")
+    assert np.array_equal(run_device(session, s, a_t.data_ptr(), m, N), got)
+    buf = torch.zeros(m * K + 1, dtype=torch.int16, device="cuda:0")
+    buf[1:] = a_t.reshape(-1)
+    if W.left_signs is not None:
+        signs = torch.zeros(gs + 1, dtype=torch.uint8, device="cuda:0")
+        signs[1:] = keep["left_signs"]
+        s.left_signs = signs.data_ptr() + 1
+    assert np.array_equal(run_device(session, s, buf.data_ptr() + 2, m, N), got)
