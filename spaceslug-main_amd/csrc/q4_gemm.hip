@@ -922,6 +922,13 @@ Q4Plan plan_q4gemm(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, ui
     if (m <= 32) {
         plan.contract_bytes = lora_bytes;
         take_digits();
+        // The decode GEMV, after a launch for T, where it saves more over the digit kernel than its epilogue
+        // costs (us per call, digit kernel and GEMV: 1 x 4096 -> 4096 rank 8 15.0, 11.0; 1 x 14336 -> 4096 rank 16
+        // 29.7, 19.5; 2 x 4096 -> 2048 rank 32 16.1, 13.8; but 1 x 1024 -> 8192 rank 32 12.2, 12.3; 1 x 512 -> 14336
+        // rank 16 11.8, 12.7; 2 x 2048 -> 2048 rank 64 13.6, 14.1) and the digit kernel needs that launch too
+        // (1 x 2048 -> 1000 rank 2 9.2 without it, 10.0 on the GEMV).
+        if (plan.t_splits > 0 && gemv_takes(m, k) && k > 1024 && (m == 1 || rank <= 32 || k >= 4096))
+            plan.kind = Q4Plan::kGemv;
         return plan;
     }
     plan.kind = Q4Plan::kWide;
@@ -972,6 +979,9 @@ hipError_t launch_q4gemm(const Q4Plan& plan, const DeviceInfo& dev, const float*
                          const uint8_t* w_packed, const float* w_scales, float* y, uint32_t m,
                          uint32_t n, uint32_t k, const float* la, const float* lb, uint32_t rank,
                          float lora_scale, void* workspace, hipStream_t stream) {
+    if (plan.kind == Q4Plan::kGemv && rank > 0)
+        return launch_gemv_lora(dev, x, w_packed, w_scales, y, m, n, k, la, lb, rank, lora_scale, plan.t_splits,
+                                static_cast<float*>(workspace), stream);
     if (plan.kind == Q4Plan::kGemv) return launch_gemv(dev, x, w_packed, w_scales, y, m, n, k, stream);
     if (plan.kind == Q4Plan::kDigits)
         return launch_q4gemm_small(dev, x, w_packed, w_scales, y, m, n, k, la, lb, rank, lora_scale, plan.t_splits, plan.tiles,

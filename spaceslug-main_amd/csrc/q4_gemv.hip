@@ -19,6 +19,7 @@
 // (q4_small.hip), which forms its group sums the same exact way on the int8 matrix cores.
 #include "q4_device.hpp"
 #include "q4_kernels.hpp"
+#include "q4_lora.hpp"
 
 #include <algorithm>
 
@@ -238,15 +239,83 @@ __device__ __forceinline__ double pipe_partial(const PipeSlot<SPC>& slot, const 
     return acc;
 }
 
+// LoRA term of a decode call: T's partials (lora_t_block, [t_splits][MR][rank]) from the launch before.
+// 1 x 4096 -> 4096 rank 8: 15.0 us on the digit kernel, 11.0 here (4.0 without LoRA); two launches and the
+// latency of T's and then lb's loads at the end bound it.
+struct GemvLora {
+    const float* tpart;
+    const float* lb;
+    int t_splits, rank;
+    float scale;
+};
+
+// Lane l gets T[row][l] for l < rank (rank <= 64). Partials are loaded, at most 8 of a row (K <= 4096), and
+// summed, in double and in order, in two steps, so that the sums wait for nothing; more take rounds.
+template <int MR>
+struct GemvLoraT {
+    float p[MR][kLoraTRound];
+};
+template <int MR>
+__device__ __forceinline__ void gemv_lora_load(const GemvLora& lora, int lane, GemvLoraT<MR>& t) {
+    const size_t plane = static_cast<size_t>(MR) * lora.rank;
+#pragma unroll
+    for (int r = 0; r < MR; ++r)
+#pragma unroll
+        for (int z = 0; z < kLoraTRound; ++z)
+            t.p[r][z] = lora.tpart[min(z, lora.t_splits - 1) * plane + r * lora.rank + min(lane, lora.rank - 1)];
+}
+template <int MR>
+__device__ __forceinline__ void gemv_lora_sum(const GemvLora& lora, const GemvLoraT<MR>& t, float (&out)[MR]) {
+#pragma unroll
+    for (int r = 0; r < MR; ++r) {
+        double sum = 0.0;
+#pragma unroll
+        for (int z = 0; z < kLoraTRound; ++z)
+            if (z < lora.t_splits) sum += static_cast<double>(t.p[r][z]);
+        out[r] = static_cast<float>(sum);
+    }
+}
+template <int MR>
+__device__ __forceinline__ void gemv_lora_t(const GemvLora& lora, int lane, float (&t)[MR]) {
+#pragma unroll
+    for (int r = 0; r < MR; ++r) {
+        float v[1];
+        lora_t_values<1>(lora.tpart, lora.t_splits, MR, lora.rank, 0, lora.rank, r, lane, 0, lora.rank, v);
+        t[r] = v[0];
+    }
+}
+
+// s[row] += scale * sum_r T[row][r] * lb[r][n] in double, T spread over the lanes: run by the whole wavefront.
+template <int MR>
+__device__ __forceinline__ void gemv_lora_add(const GemvLora& lora, double (&s)[MR], const float (&t)[MR], int N, int n) {
+    constexpr int kRound = 16;
+    double tb[MR] = {};
+    for (int r0 = 0; r0 < lora.rank; r0 += kRound) {
+        float b[kRound];
+#pragma unroll
+        for (int i = 0; i < kRound; ++i) b[i] = lora.lb[static_cast<size_t>(min(r0 + i, lora.rank - 1)) * N + n];
+#pragma unroll
+        for (int i = 0; i < kRound; ++i)
+            if (r0 + i < lora.rank)
+#pragma unroll
+                for (int r = 0; r < MR; ++r)
+                    tb[r] = fma(static_cast<double>(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(t[r]), r0 + i))),
+                                static_cast<double>(b[i]), tb[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < MR; ++r) s[r] = fma(static_cast<double>(lora.scale), tb[r], s[r]);
+}
+
 // Columns col0 .. col0 + cpb - 1 of a row x holding an infinity or a NaN, in double
 // with every term x * (v * s) formed as the double reference forms it (q4gemm_ref,
 // test_q4gemm.cpp:102-119): such a row's outputs are all infinite or NaN, and IEEE
 // arithmetic gives the reference's pattern (inf * 0 is NaN, opposite infinities give
 // NaN) in any summation order. Lane l takes groups l, l + 64, ...; reached only for
 // non-finite x, so it is written for clarity, not speed.
+template <class... Lora>
 __device__ __forceinline__ void pipe_ieee_columns(const float* x, const uint32_t* __restrict__ wq,
                                                const float* __restrict__ ws, float* __restrict__ y, int N, int G,
-                                               int col0, int cpb, int lane) {
+                                               int col0, int cpb, int lane, float lora_t, const Lora&... lora) {
     for (int i = 0; i < cpb && col0 + i < N; ++i) {
         const int col = col0 + i;
         double acc = 0.0;
@@ -261,15 +330,22 @@ __device__ __forceinline__ void pipe_ieee_columns(const float* x, const uint32_t
             }
         }
         for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+        if constexpr (sizeof...(Lora) > 0) {
+            double sum[1] = {acc};
+            const float t[1] = {lora_t};
+            gemv_lora_add<1>(lora..., sum, t, N, col);
+            acc = sum[0];
+        }
         if (lane == 0) y[col] = static_cast<float>(acc);
     }
 }
 
-template <int SPC, int D, int MR>
+template <int SPC, int D, int MR, class... Lora>
 __global__ __launch_bounds__(kGemvThreads) void q4_gemv_pipe_kernel(const float* x,  // not restrict: x loads stay ahead of the weights
                                                                    const u32x4* __restrict__ wq,
                                                                    const float* __restrict__ ws,
-                                                                   float* __restrict__ y, int N, int K, int reps) {
+                                                                   float* __restrict__ y, int N, int K, int reps,
+                                                                   Lora... lora) {
     constexpr int S = D + 1;                      // register slots
     constexpr int kGroups = 64 * SPC;             // groups per lane pass: K <= 32 * kGroups
     constexpr int kRecoded = kGemvThreads / 2;    // groups recoded (two threads per group)
@@ -284,6 +360,9 @@ __global__ __launch_bounds__(kGemvThreads) void q4_gemv_pipe_kernel(const float*
     const int cpb = D + S * reps;  // columns per wavefront (<= 64)
     const int col0 = wave * cpb;
     const int G = K >> 5;
+    [[maybe_unused]] float lora_t[MR] = {};
+    [[maybe_unused]] GemvLoraT<MR> lora_p;
+    if constexpr (sizeof...(Lora) > 0) gemv_lora_load<MR>(lora..., lane, lora_p);
 
     // x first (thread t recodes half t & 1, 16 values, of group t >> 1 of every row), then the
     // first D columns, all before any wait.
@@ -343,9 +422,11 @@ __global__ __launch_bounds__(kGemvThreads) void q4_gemv_pipe_kernel(const float*
         for (int s = 0; s < SPC; ++s) nonfinite = nonfinite || __builtin_isnan(xd[r].c[s]);
     if (__builtin_amdgcn_ballot_w64(nonfinite) != 0) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the prologue's column loads
+        if constexpr (sizeof...(Lora) > 0) gemv_lora_sum<MR>(lora..., lora_p, lora_t);
+#pragma unroll
         for (int r = 0; r < MR; ++r)
             pipe_ieee_columns(x + static_cast<size_t>(r) * K, reinterpret_cast<const uint32_t*>(wq), ws,
-                              y + static_cast<size_t>(r) * N, N, G, col0, cpb, lane);
+                              y + static_cast<size_t>(r) * N, N, G, col0, cpb, lane, lora_t[r], lora...);
         return;
     }
 
@@ -354,9 +435,10 @@ __global__ __launch_bounds__(kGemvThreads) void q4_gemv_pipe_kernel(const float*
     // between its own issue points: interleaved slots would make the wavefront wait for every
     // outstanding load first. (Reducing four columns at once with fewer instructions
     // measured slower: the wavefront then waits out one long dependent chain per four.)
-    float result[MR];
+    using Sum = std::conditional_t<(sizeof...(Lora) > 0), double, float>;  // rounded once, after the LoRA term
+    Sum result[MR];
 #pragma unroll
-    for (int r = 0; r < MR; ++r) result[r] = 0.0f;
+    for (int r = 0; r < MR; ++r) result[r] = 0;
     for (int rep = 0; rep < reps; ++rep) {
 #pragma unroll
         for (int s = 0; s < S; ++s) {
@@ -365,7 +447,7 @@ __global__ __launch_bounds__(kGemvThreads) void q4_gemv_pipe_kernel(const float*
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int r = 0; r < MR; ++r) {
-                const float t = static_cast<float>(wave_reduce_dpp(pipe_partial<SPC>(slot[s], xd[r])));
+                const Sum t = static_cast<Sum>(wave_reduce_dpp(pipe_partial<SPC>(slot[s], xd[r])));
                 result[r] = lane == i ? t : result[r];
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -377,14 +459,18 @@ __global__ __launch_bounds__(kGemvThreads) void q4_gemv_pipe_kernel(const float*
         const int i = reps * S + s;
 #pragma unroll
         for (int r = 0; r < MR; ++r) {
-            const float t = static_cast<float>(wave_reduce_dpp(pipe_partial<SPC>(slot[s], xd[r])));
+            const Sum t = static_cast<Sum>(wave_reduce_dpp(pipe_partial<SPC>(slot[s], xd[r])));
             result[r] = lane == i ? t : result[r];
         }
+    }
+    if constexpr (sizeof...(Lora) > 0) {
+        gemv_lora_sum<MR>(lora..., lora_p, lora_t);
+        gemv_lora_add<MR>(lora..., result, lora_t, N, min(col0 + lane, N - 1));
     }
     // lane c holds column col0 + c: one coalesced store of the wavefront's run per row
     if (lane < cpb && col0 + lane < N)
 #pragma unroll
-        for (int r = 0; r < MR; ++r) y[static_cast<size_t>(r) * N + col0 + lane] = result[r];
+        for (int r = 0; r < MR; ++r) y[static_cast<size_t>(r) * N + col0 + lane] = static_cast<float>(result[r]);
 }
 
 // Unit i of a column set of the K-split kernel: column col0 + i, groups gb .. gb + gn - 1. A unit
@@ -416,12 +502,12 @@ __device__ __forceinline__ void pipe_issue_unit(PipeSlot<SPC>& slot, const u32x4
 // one row, K = 14336, N = 4096, 64 weight copies, four wavefronts per column took 10.7 us per launch in
 // workgroups of 256 threads, 9.6 in 512 and 9.6-9.7 in 1024 (D = 2); D = 6 at 256 threads 11.4;
 // waiting for x before issuing the first units changed nothing.
-template <int SPC, int D, int KZ, int THREADS, int MR>
+template <int SPC, int D, int KZ, int THREADS, int MR, class... Lora>
 __global__ __launch_bounds__(THREADS) void q4_gemv_split_kernel(const float* x,  // not restrict, as above
                                                                const u32x4* __restrict__ wq,
                                                                const float* __restrict__ ws,
                                                                float* __restrict__ y, int N, int K, int cols,
-                                                               int reps) {
+                                                               int reps, Lora... lora) {
     constexpr int S = D + 1;
     constexpr int kWaves = THREADS >> 6;
     constexpr int kSets = kWaves / KZ;                        // column sets per workgroup
@@ -439,6 +525,9 @@ __global__ __launch_bounds__(THREADS) void q4_gemv_split_kernel(const float* x, 
     const int G = K >> 5;
     const int gb = z * G / KZ;
     const int gn = (z + 1) * G / KZ - gb;
+    [[maybe_unused]] float lora_t[MR] = {};
+    if constexpr (sizeof...(Lora) > 0)
+        if (z == 0) gemv_lora_t<MR>(lora..., lane, lora_t);
 
     // x first (every row's and pass's loads, groups past G clamped to the last), then the first D
     // units.
@@ -487,9 +576,10 @@ __global__ __launch_bounds__(THREADS) void q4_gemv_split_kernel(const float* x, 
     if (__builtin_amdgcn_ballot_w64(nonfinite) != 0) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the prologue's column loads
         if (z == 0)
+#pragma unroll
             for (int r = 0; r < MR; ++r)
                 pipe_ieee_columns(x + static_cast<size_t>(r) * K, reinterpret_cast<const uint32_t*>(wq), ws,
-                                  y + static_cast<size_t>(r) * N, N, G, col0, cols, lane);
+                                  y + static_cast<size_t>(r) * N, N, G, col0, cols, lane, lora_t[r], lora...);
         return;
     }
     // The lane's groups gb + l and gb + 64 + l. Entries past the part (the next part's groups, or
@@ -549,14 +639,18 @@ __global__ __launch_bounds__(THREADS) void q4_gemv_split_kernel(const float* x, 
 #pragma unroll
     for (int r = 0; r < MR; ++r) part[wb][r][lane] = result[r];
     __syncthreads();
-    if (z == 0 && lane < cols && col0 + lane < N)
+    if (z != 0) return;
+    double sum[MR];
 #pragma unroll
-        for (int r = 0; r < MR; ++r) {
-            double t = part[wb][r][lane];
+    for (int r = 0; r < MR; ++r) {
+        sum[r] = part[wb][r][lane];
 #pragma unroll
-            for (int q = 1; q < KZ; ++q) t += part[wb + q][r][lane];
-            y[static_cast<size_t>(r) * N + col0 + lane] = static_cast<float>(t);
-        }
+        for (int q = 1; q < KZ; ++q) sum[r] += part[wb + q][r][lane];
+    }
+    if constexpr (sizeof...(Lora) > 0) gemv_lora_add<MR>(lora..., sum, lora_t, N, min(col0 + lane, N - 1));
+    if (lane < cols && col0 + lane < N)
+#pragma unroll
+        for (int r = 0; r < MR; ++r) y[static_cast<size_t>(r) * N + col0 + lane] = static_cast<float>(sum[r]);
 }
 
 }  // namespace
@@ -572,9 +666,9 @@ __global__ __launch_bounds__(THREADS) void q4_gemv_split_kernel(const float* x, 
 // 2 x 4096 -> 14336 takes 11.5 us against 14.8 for the small-batch GEMM (2 x 2048 -> 4096: 4.5
 // against 5.7 us). One lane slot at K <= 2048 keeps half the lanes from computing on zeros:
 // 1 x 2048 -> 14336 5.4 us against 6.8.
-template <int MR>
+template <int MR, class... Lora>
 static hipError_t launch_gemv_pipelined(const DeviceInfo& dev, const float* x, const uint8_t* w_packed,
-                                 const float* w_scales, float* y, uint32_t n, uint32_t k, hipStream_t stream) {
+                                 const float* w_scales, float* y, uint32_t n, uint32_t k, hipStream_t stream, Lora... lora) {
     constexpr int D = 4, S = D + 1, kMaxReps = (64 - D) / S;
     const size_t waves_per_block = kGemvThreads / 64;
     const size_t slots = static_cast<size_t>(dev.cu_count) * waves_per_block;  // wavefronts in one round
@@ -584,13 +678,13 @@ static hipError_t launch_gemv_pipelined(const DeviceInfo& dev, const float* x, c
     const size_t waves = (static_cast<size_t>(n) + cpb - 1) / cpb;
     const size_t blocks = (waves + waves_per_block - 1) / waves_per_block;
     if (k / kGroup <= 64u)  // one group per lane: no idle second slot
-        hipLaunchKernelGGL((q4_gemv_pipe_kernel<1, D, MR>), dim3(static_cast<unsigned>(blocks)), dim3(kGemvThreads), 0,
+        hipLaunchKernelGGL((q4_gemv_pipe_kernel<1, D, MR, Lora...>), dim3(static_cast<unsigned>(blocks)), dim3(kGemvThreads), 0,
                            stream, x, reinterpret_cast<const u32x4*>(w_packed), w_scales, y, static_cast<int>(n),
-                           static_cast<int>(k), reps);
+                           static_cast<int>(k), reps, lora...);
     else
-        hipLaunchKernelGGL((q4_gemv_pipe_kernel<2, D, MR>), dim3(static_cast<unsigned>(blocks)), dim3(kGemvThreads), 0,
+        hipLaunchKernelGGL((q4_gemv_pipe_kernel<2, D, MR, Lora...>), dim3(static_cast<unsigned>(blocks)), dim3(kGemvThreads), 0,
                            stream, x, reinterpret_cast<const u32x4*>(w_packed), w_scales, y, static_cast<int>(n),
-                           static_cast<int>(k), reps);
+                           static_cast<int>(k), reps, lora...);
     return hipGetLastError();
 }
 
@@ -599,9 +693,9 @@ static hipError_t launch_gemv_pipelined(const DeviceInfo& dev, const float* x, c
 // column sets (two for KZ = 2, whose smaller sets would leave the pipeline too short at N = 4096;
 // one for KZ = 8): 256, 768, 1024 or 512 threads. Columns per set: the fewest whose workgroups all
 // fit on the CUs at once (at most 64).
-template <int D, int KZ, int THREADS, int MR = 1, int SPC = 2>
+template <int D, int KZ, int THREADS, int MR = 1, int SPC = 2, class... Lora>
 static hipError_t launch_gemv_split(const DeviceInfo& dev, const float* x, const uint8_t* w_packed,
-                                    const float* w_scales, float* y, uint32_t n, uint32_t k, hipStream_t stream) {
+                                    const float* w_scales, float* y, uint32_t n, uint32_t k, hipStream_t stream, Lora... lora) {
     constexpr int S = D + 1;
     constexpr size_t kSets = (THREADS / 64) / KZ;
     const size_t slots = static_cast<size_t>(dev.cu_count) * kSets;  // column sets in one round
@@ -609,19 +703,19 @@ static hipError_t launch_gemv_split(const DeviceInfo& dev, const float* x, const
     const int reps = cols > static_cast<size_t>(D) ? static_cast<int>((cols - D + S - 1) / S) : 0;
     const size_t sets = (n + cols - 1) / cols;
     const size_t blocks = (sets + kSets - 1) / kSets;
-    hipLaunchKernelGGL((q4_gemv_split_kernel<SPC, D, KZ, THREADS, MR>), dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0,
+    hipLaunchKernelGGL((q4_gemv_split_kernel<SPC, D, KZ, THREADS, MR, Lora...>), dim3(static_cast<unsigned>(blocks)), dim3(THREADS), 0,
                        stream, x, reinterpret_cast<const u32x4*>(w_packed), w_scales, y, static_cast<int>(n),
-                       static_cast<int>(k), static_cast<int>(cols), reps);
+                       static_cast<int>(k), static_cast<int>(cols), reps, lora...);
     return hipGetLastError();
 }
 
-hipError_t launch_gemv(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
-                       float* y, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream) {
-    if (!gemv_takes(m, k)) return hipErrorInvalidValue;
+template <class... Lora>
+static hipError_t dispatch_gemv(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
+                                float* y, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream, Lora... lora) {
     const uint32_t groups = k / kGroup;
     if (m == 2) {
         if (groups <= static_cast<uint32_t>(kGemvPipeMaxGroups))
-            return launch_gemv_pipelined<2>(dev, x, w_packed, w_scales, y, n, k, stream);
+            return launch_gemv_pipelined<2>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
         // Two rows' digits of two groups per lane take 128 registers, so the K-split forms run at
         // most two wavefronts per SIMD (up to K = 8192 two, against one in the one-row form:
         // 2 x 8192 -> 14336 20.4 against 22.4 us); between K = 8192 and 12288, where four parts of two
@@ -630,17 +724,33 @@ hipError_t launch_gemv(const DeviceInfo& dev, const float* x, const uint8_t* w_p
         // against 10.0 and 17.1 against 15.4 us). Up to K = 4096 the one-wavefront kernel beats the
         // K-split one at two wavefronts per SIMD (2 x 4096 -> 14336: 11.5 against 12.3 us).
         if (groups <= 2u * kGemvPipeMaxGroups)
-            return launch_gemv_split<4, 2, 512, 2>(dev, x, w_packed, w_scales, y, n, k, stream);
+            return launch_gemv_split<4, 2, 512, 2, 2>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
         if (groups <= 3u * kGemvPipeMaxGroups)
-            return launch_gemv_split<3, 6, 768, 2, 1>(dev, x, w_packed, w_scales, y, n, k, stream);
-        return launch_gemv_split<3, 4, 512, 2>(dev, x, w_packed, w_scales, y, n, k, stream);
+            return launch_gemv_split<3, 6, 768, 2, 1>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
+        return launch_gemv_split<3, 4, 512, 2, 2>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
     }
     if (groups <= static_cast<uint32_t>(kGemvPipeMaxGroups))
-        return launch_gemv_pipelined<1>(dev, x, w_packed, w_scales, y, n, k, stream);
-    if (groups <= 2u * kGemvPipeMaxGroups) return launch_gemv_split<4, 2, 256>(dev, x, w_packed, w_scales, y, n, k, stream);
-    if (groups <= 3u * kGemvPipeMaxGroups) return launch_gemv_split<2, 3, 768>(dev, x, w_packed, w_scales, y, n, k, stream);
-    if (groups <= 4u * kGemvPipeMaxGroups) return launch_gemv_split<2, 4, 1024>(dev, x, w_packed, w_scales, y, n, k, stream);
-    return launch_gemv_split<4, 8, 512>(dev, x, w_packed, w_scales, y, n, k, stream);
+        return launch_gemv_pipelined<1>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
+    if (groups <= 2u * kGemvPipeMaxGroups) return launch_gemv_split<4, 2, 256>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
+    if (groups <= 3u * kGemvPipeMaxGroups) return launch_gemv_split<2, 3, 768>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
+    if (groups <= 4u * kGemvPipeMaxGroups) return launch_gemv_split<2, 4, 1024>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
+    return launch_gemv_split<4, 8, 512>(dev, x, w_packed, w_scales, y, n, k, stream, lora...);
+}
+
+hipError_t launch_gemv(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
+                       float* y, uint32_t m, uint32_t n, uint32_t k, hipStream_t stream) {
+    if (!gemv_takes(m, k)) return hipErrorInvalidValue;
+    return dispatch_gemv(dev, x, w_packed, w_scales, y, m, n, k, stream);
+}
+
+hipError_t launch_gemv_lora(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
+                            float* y, uint32_t m, uint32_t n, uint32_t k, const float* la, const float* lb, uint32_t rank,
+                            float lora_scale, int t_splits, float* tpart, hipStream_t stream) {
+    if (!gemv_takes(m, k)) return hipErrorInvalidValue;
+    const hipError_t e = launch_lora_t(x, la, tpart, m, k, rank, t_splits, stream);
+    if (e != hipSuccess) return e;
+    return dispatch_gemv(dev, x, w_packed, w_scales, y, m, n, k, stream,
+                         GemvLora{tpart, lb, t_splits, static_cast<int>(rank), lora_scale});
 }
 
 }  // namespace spaceslug

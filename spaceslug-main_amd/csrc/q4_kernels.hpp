@@ -33,7 +33,7 @@ constexpr bool gemv_takes(uint32_t m, uint32_t k) {
 
 // Launch shape chosen by plan_q4gemm for one call.
 struct Q4Plan {
-    // kGemv: decode GEMV (gemv_takes, no LoRA); kDigits: every other call up to 32 rows, and taller
+    // kGemv: decode GEMV (gemv_takes); kDigits: every other call up to 32 rows, and taller
     // ones whose estimate is the lowest, exact integer group sums on the int8 matrix cores
     // (q4_small.hip); kWide: m > 32; kMid: m > 32 without LoRA whose 128 x 128 grid would need a
     // K-split while its 64 x 64 grid fits the CUs once (k % 64 == 0, k <= 4096).
@@ -58,7 +58,7 @@ Q4Plan plan_q4gemm(const DeviceInfo& dev, uint32_t m, uint32_t n, uint32_t k, ui
 // Kernel launches of launch_q4gemm for a plan.
 constexpr int plan_launches(const Q4Plan& p) {
     switch (p.kind) {
-        case Q4Plan::kGemv: return 1;
+        case Q4Plan::kGemv:
         case Q4Plan::kDigits: return p.t_splits > 0 ? 2 : 1;
         case Q4Plan::kMid: return 2;
         default: return p.splits > 1 ? 3 : 2;
@@ -69,6 +69,16 @@ constexpr int plan_launches(const Q4Plan& p) {
 hipError_t launch_gemv(const DeviceInfo& dev, const float* x, const uint8_t* w_packed,
                        const float* w_scales, float* y, uint32_t m, uint32_t n, uint32_t k,
                        hipStream_t stream);
+
+// The same with the LoRA term scale * (x * la) * lb: T's partials (tpart, t_splits * m * rank floats) in a
+// launch of their own first.
+hipError_t launch_gemv_lora(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
+                            float* y, uint32_t m, uint32_t n, uint32_t k, const float* la, const float* lb, uint32_t rank,
+                            float lora_scale, int t_splits, float* tpart, hipStream_t stream);
+
+// T = x * la as t_splits partials [t_splits][m][rank], for the kernels up to 32 rows (q4_small.hip).
+hipError_t launch_lora_t(const float* x, const float* la, float* tpart, uint32_t m, uint32_t k, uint32_t rank,
+                         int t_splits, hipStream_t stream);
 
 // y = x * dequant(W) [+ scale * (x * la) * lb]. `workspace` must hold
 // plan.workspace_bytes bytes (may be null when that is 0).

@@ -811,6 +811,15 @@ DigitTiles plan_digit_tiles(const DeviceInfo& dev, uint32_t m, uint32_t n, uint3
     return {tiles, us};
 }
 
+hipError_t launch_lora_t(const float* x, const float* la, float* tpart, uint32_t m, uint32_t k, uint32_t rank,
+                         int t_splits, hipStream_t stream) {
+    const int tiles_m = static_cast<int>((m + 15) / 16), tiles_r = static_cast<int>((rank + 15) / 16);
+    hipLaunchKernelGGL(small_lora_prep_kernel, dim3(static_cast<unsigned>(tiles_m * tiles_r * t_splits)), dim3(256), 0,
+                       stream, x, la, tpart, static_cast<int>(m), static_cast<int>(k), static_cast<int>(rank), tiles_m,
+                       tiles_r);
+    return hipGetLastError();
+}
+
 hipError_t launch_q4gemm_small(const DeviceInfo& dev, const float* x, const uint8_t* w_packed, const float* w_scales,
                                float* y, uint32_t m, uint32_t n, uint32_t k, const float* la, const float* lb,
                                uint32_t rank, float lora_scale, int t_splits, int tiles, void* workspace,
@@ -825,10 +834,7 @@ hipError_t launch_q4gemm_small(const DeviceInfo& dev, const float* x, const uint
     const int W = total <= static_cast<size_t>(dev.cu_count) ? 16 : total <= 2 * static_cast<size_t>(dev.cu_count) ? 8 : 4;
     if (t_splits > 0) {
         tpart = static_cast<float*>(workspace);
-        const int tiles_m_t = (M + 15) / 16, tiles_r = (R + 15) / 16;
-        hipLaunchKernelGGL(small_lora_prep_kernel, dim3(static_cast<unsigned>(tiles_m_t * tiles_r * t_splits)),
-                           dim3(256), 0, stream, x, la, tpart, M, K, R, tiles_m_t, tiles_r);
-        const hipError_t pe = hipGetLastError();
+        const hipError_t pe = launch_lora_t(x, la, tpart, m, k, rank, t_splits, stream);
         if (pe != hipSuccess) return pe;
     }
     const float* lbp = rank ? lb : nullptr;
