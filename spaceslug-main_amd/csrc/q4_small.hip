@@ -191,7 +191,8 @@ __device__ float ieee_row_value(const float* x, const uint32_t* wq, const float*
 // NI: output register pairs per lane in use (rows 2 i + h, i < NI): 1 for M <= 2, 2 for M <= 4,
 // else 4. W: wavefronts per workgroup, splitting K. Every variant keeps four wavefronts per SIMD
 // resident (at most 128 VGPRs and 40 KiB of LDS per wavefront), which hides the recoding's
-// dependent chains. OWN_T: a LoRA call whose T the workgroup computes itself. Taken for short K and for some grids of one tile per CU (plan_digit_tiles).
+// dependent chains. OWN_T: a LoRA call whose T the workgroup computes itself (short K). Taken for short K and
+// for some grids of one tile per CU (plan_digit_tiles).
 template <int NI, int W, bool OWN_T>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(4))) void q4_gemm_small_kernel(const float* x, const uint32_t* wq, const float* ws,
                                                                float* __restrict__ y, int M, int N, int K, int RB,
